@@ -126,9 +126,9 @@ int gpuq_hessian_accumulate_dev(const float *d_X, int64_t nrows, int64_t ne0, do
  * n inputs; not modified) -> d_U [ne0][ne0] f64 (device, row-major upper factor: U^T U = the inverse of the damped,
  * normalized, block-permuted Hessian, with the reference's dead-column rule and its one retry with 10x more ridge),
  * perm [ne0] (host: the column permutation, whole 256-column blocks; order 0 'seq', 1 'act'), diag_n [ne0] (host,
- * diag(H)/n permuted; may be NULL) and dead [ne0] (host flags, original order; may be NULL). Uses rocSOLVER's potrf /
- * potri (loaded on first use). Returns 0; 1 bad arguments (ne0 a multiple of 256, at most 65280), 2 rocBLAS or
- * rocSOLVER not loadable, 3 not positive definite, 4 a HIP error. Synchronizes `stream`. */
+ * diag(H)/n permuted; may be NULL) and dead [ne0] (host flags, original order; may be NULL).
+ * Returns 0; 1 bad arguments (ne0 a multiple of 256, at most 65280), 3 not positive definite, 4 a HIP error.
+ * Synchronizes `stream`. */
 int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n, double damp, int order, double *d_U,
                              int64_t *perm, double *diag_n, unsigned char *dead, void *stream);
 

@@ -4,10 +4,7 @@
 // The exported functions keep the reference library's signatures, return conventions and table file format
 // (gpuq/gpuq.hip:2059-2328 of the reference), so its Python drivers load this library unchanged; they are declared
 // with their reference counterparts in include/gpuq.h.
-#include <dlfcn.h>
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <cstdio>
 #include <cstring>
@@ -29,6 +26,7 @@
 #include "dequant.cuh"
 #include "ldlq.cuh"
 #include "hessian.cuh"
+#include "chol.cuh"
 
 extern "C" size_t gpuq_block_bytes(int type);
 
@@ -1035,34 +1033,26 @@ extern "C" size_t gpuq_ldlq_dev_noalloc(int type, float *d_wp, const double *d_u
 // ------------------------------------------------------------------ the Hessian preparation and the host LDLQ loop
 namespace {
 
-// rocBLAS / rocSOLVER, opened on first use (the quantizer never needs them): the copies the process already loaded
-// when the caller's framework brought them (same sonames), else ROCm's
-struct Lapack {
-    bool tried = false, ok = false;
-    decltype(&rocblas_create_handle) create = nullptr;
-    decltype(&rocblas_set_stream) set_stream = nullptr;
-    decltype(&rocsolver_dpotrf) potrf = nullptr;
-    decltype(&rocsolver_dpotri) potri = nullptr;
-    rocblas_handle h = nullptr;
-};
-Lapack g_lp;
-std::mutex g_mu_h;   // the Hessian preparation's handle and buffers
+std::mutex g_mu_h;   // the Hessian preparation's buffer
 Buf g_hd;            // device: diag (f64) | perm (i64) | dead (u8) | factorization info
 
-bool lapack_ready() {
-    if (g_lp.tried) return g_lp.ok;
-    g_lp.tried = true;
-    void *blas = dlopen("librocblas.so.5", RTLD_NOW | RTLD_GLOBAL);
-    void *sol = dlopen("librocsolver.so.0", RTLD_NOW | RTLD_GLOBAL);
-    if (!blas || !sol) return false;
-    g_lp.create = (decltype(g_lp.create))dlsym(blas, "rocblas_create_handle");
-    g_lp.set_stream = (decltype(g_lp.set_stream))dlsym(blas, "rocblas_set_stream");
-    g_lp.potrf = (decltype(g_lp.potrf))dlsym(sol, "rocsolver_dpotrf");
-    g_lp.potri = (decltype(g_lp.potri))dlsym(sol, "rocsolver_dpotri");
-    if (!g_lp.create || !g_lp.set_stream || !g_lp.potrf || !g_lp.potri) return false;
-    if (hipSetDevice(g_device) != hipSuccess || g_lp.create(&g_lp.h) != rocblas_status_success) return false;
-    g_lp.ok = true;
-    return true;
+// U (chol.cuh) in place of the permuted Hessian A (its upper triangle), launches only; *d_info (zeroed by the caller)
+// becomes 1 when A is not positive definite
+void launch_factor(double *A, int64_t n, int *d_info, hipStream_t st) {
+    const int64_t nb = n / CH_NB;
+    hipLaunchKernelGGL(k_chol_last, dim3(1), dim3(256), 0, st, A, n, d_info);
+    for (int64_t k = nb - 1; k > 0; --k) {
+        hipLaunchKernelGGL(k_chol_panel, dim3((unsigned)(k * CH_NB / 32)), dim3(256), 0, st, A, n, k);
+        const int64_t nt = k * (k + 1) / 2 - 1;          // the tiles beside (k-1, k-1), in whole rounds of the 8 XCDs
+        hipLaunchKernelGGL(k_chol_update, dim3((unsigned)(1 + (nt + 7) / 8 * 8)), dim3(256), 0, st, A, n, k, d_info);
+    }
+    for (int64_t s = 1; s < nb; s *= 2) {
+        const int64_t pairs = (nb - s + 2 * s - 1) / (2 * s), t = s * (CH_NB / CHT);
+        const dim3 grid((unsigned)(t * t), (unsigned)pairs);
+        hipLaunchKernelGGL(k_tri_mul1, grid, dim3(256), 0, st, A, n, s);
+        hipLaunchKernelGGL(k_tri_mul2, grid, dim3(256), 0, st, A, n, s);
+    }
+    hipLaunchKernelGGL(k_zero_lower, dim3((unsigned)((n + 255) / 256), (unsigned)n), dim3(256), 0, st, A, n);
 }
 
 // a factorization's info (0: done; > 0: not positive definite), -1 when it cannot be read
@@ -1100,15 +1090,13 @@ extern "C" int gpuq_hessian_accumulate_dev(const float *d_X, int64_t nrows, int6
 // rows; one retry with 10x more ridge when Hp does not factor), and on the host perm (ne0 column indices, whole
 // 256-blocks: order 0 'seq' keeps them in order, 1 'act' sorts them by descending energy, ties in order), diag_n
 // (diag(Hn)[perm]) and dead (ne0 flags, original order); either of the last two may be NULL. Returns 0, or 1 for bad
-// arguments, 2 when rocBLAS / rocSOLVER cannot be loaded, 3 when the matrix does not factor, 4 on a HIP error.
+// arguments, 3 when the matrix does not factor, 4 on a HIP error.
 extern "C" int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n, double damp, int order, double *d_U,
                                         int64_t *perm, double *diag_n, uint8_t *dead, void *stream) {
     if (g_device < 0 || !d_H || !d_U || !perm || ne0 <= 0 || ne0 % QK || ne0 > 65535) return 1;   // (grid rows)
     if ((order != 0 && order != 1) || !(damp >= 0) || ((uintptr_t)d_H & 7) || ((uintptr_t)d_U & 7)) return 1;
     std::lock_guard<std::mutex> lock(g_mu_h);
-    if (!lapack_ready()) return 2;
     const hipStream_t st = (hipStream_t)stream;
-    if (g_lp.set_stream(g_lp.h, st) != rocblas_status_success) return 4;
     const size_t o_perm = (size_t)ne0 * 8, o_dead = o_perm + (size_t)ne0 * 8, o_info = (o_dead + ne0 + 15) & ~15ull;
     if (!g_hd.grow(o_info + 16)) return 4;
     double *dd = (double *)g_hd.p;
@@ -1151,27 +1139,18 @@ extern "C" int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n
         hipMemcpyAsync(dz, zd.data(), (size_t)ne0, hipMemcpyHostToDevice, st) != hipSuccess)
         return 4;
     const double r1 = damp * mean;
-    const rocblas_int nn = (rocblas_int)ne0;
-    hipLaunchKernelGGL(k_hess_perm, g2, dim3(256), 0, st, d_H, ne0, nd, (const int64_t *)dp, (const uint8_t *)dz, r1,
-                       d_U);
-    if (g_lp.potrf(g_lp.h, rocblas_fill_lower, nn, d_U, nn, dinfo) != rocblas_status_success) return 4;
-    int info = read_info(dinfo, st);
-    if (info > 0) {                                       // more ridge until it factors
-        hipLaunchKernelGGL(k_hess_perm, g2, dim3(256), 0, st, d_H, ne0, nd, (const int64_t *)dp,
-                           (const uint8_t *)dz, r1, d_U);
-        hipLaunchKernelGGL(k_diag_add, dim3(g1), dim3(256), 0, st, d_U, ne0, 10 * damp * mean);
-        if (g_lp.potrf(g_lp.h, rocblas_fill_lower, nn, d_U, nn, dinfo) != rocblas_status_success) return 4;
+    int info = 0;
+    for (int tries = 0; tries < 2; ++tries) {             // (the second: more ridge until it factors)
+        hipLaunchKernelGGL(k_hess_perm, g2, dim3(256), 0, st, d_H, ne0, nd, (const int64_t *)dp, (const uint8_t *)dz, r1,
+                           d_U);
+        if (tries) hipLaunchKernelGGL(k_diag_add, dim3(g1), dim3(256), 0, st, d_U, ne0, 10 * damp * mean);
+        hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, dinfo);
+        launch_factor(d_U, ne0, dinfo, st);
+        if (hipGetLastError() != hipSuccess) return 4;
         info = read_info(dinfo, st);
+        if (info <= 0) break;
     }
     if (info != 0) return info > 0 ? 3 : 4;
-    // Hp^-1 from the factor (lower triangle), made symmetric, then its own lower factor: read row-major, U
-    if (g_lp.potri(g_lp.h, rocblas_fill_lower, nn, d_U, nn, dinfo) != rocblas_status_success) return 4;
-    if ((info = read_info(dinfo, st)) != 0) return info > 0 ? 3 : 4;
-    hipLaunchKernelGGL(k_sym_from_lower, g2, dim3(256), 0, st, d_U, ne0);
-    if (g_lp.potrf(g_lp.h, rocblas_fill_lower, nn, d_U, nn, dinfo) != rocblas_status_success) return 4;
-    if ((info = read_info(dinfo, st)) != 0) return info > 0 ? 3 : 4;
-    hipLaunchKernelGGL(k_zero_upper, g2, dim3(256), 0, st, d_U, ne0);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return 4;
     for (int64_t i = 0; i < ne0; ++i) {
         perm[i] = pm[i];
         if (diag_n) diag_n[i] = d[pm[i]];
