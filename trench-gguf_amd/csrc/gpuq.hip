@@ -1078,9 +1078,8 @@ extern "C" int gpuq_hessian_accumulate_dev(const float *d_X, int64_t nrows, int6
     if (g_device < 0 || !d_X || !d_H || nrows <= 0 || ne0 <= 0 || ne0 % QK || ne0 > 65535) return 1;
     if (((uintptr_t)d_X & 3) || ((uintptr_t)d_H & 7)) return 1;
     const hipStream_t st = (hipStream_t)stream;
-    const unsigned nt = (unsigned)(ne0 / 128);
-    hipLaunchKernelGGL(k_xtx, dim3(nt, nt), dim3(256), 0, st, d_X, nrows, ne0, d_H);
-    hipLaunchKernelGGL(k_hess_mirror, dim3((unsigned)((ne0 + 255) / 256), (unsigned)ne0), dim3(256), 0, st, d_H, ne0);
+    const int64_t nr = ne0 / 128, nt = nr * (nr + 1) / 2;
+    hipLaunchKernelGGL(k_xtx, dim3((unsigned)((nt + 7) / 8 * 8)), dim3(256), 0, st, d_X, nrows, ne0, d_H);
     return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 

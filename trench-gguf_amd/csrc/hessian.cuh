@@ -45,18 +45,44 @@ __global__ __launch_bounds__(256) void k_gather_cols(const float *__restrict__ W
 
 // H += X^T X (tools/hessian_from_dump.py:73-79 of the reference: the Hessian sum over activation rows), X [nrows][ne0]
 // f32 row-major, H [ne0][ne0] f64; every product exact in f64 and each output an fma chain over the rows in order on
-// the f64 matrix cores. A workgroup of 4 waves owns a 128 x 128 tile of the lower triangle (grid: ne0/128 squared,
-// tiles above the diagonal exit at once); rows run in chunks of 16 staged in LDS as f64 (two buffers, one barrier a
-// chunk), the two panels of a chunk being X's columns of the tile's rows and of its columns. k_hess_mirror then copies
-// the lower triangle's tiles over the upper ones.
+// the f64 matrix cores. A workgroup of 4 waves owns a 128 x 128 tile of the lower triangle and writes its values to
+// the mirrored place too (the tiles beside the diagonal blocks; those hold both halves themselves); rows run in chunks
+// of 16 staged in LDS as f64 (two buffers, one barrier a chunk). The matrix cores bound it: a chunk's floats are read
+// before the last chunk's products and become f64 only after them, on their way into LDS (converted where they are
+// read, each chunk would wait for its loads). The 1-D grid holds the triangle's tiles alone and each XCD gets one range
+// of them (dealt row by row of a square grid the XCDs' shares differ by 28%), in groups of XTX_GM row tiles, rows
+// fastest, whose panels its L2 shares. 4096 rows of 7168 columns: 5.71 -> 3.89 ms with these and without the mirroring
+// pass (0.17 ms of it), 54 TFLOP/s of the 73 that a large f64 product reaches (the 1596 tiles are 6.2 for each CU, so
+// the last round leaves a tenth of the time idle; 128 x 64 tiles, 12.5 a CU, took 3.96 ms).
 #define XTX_BK 16
 #define XTX_LDS_ROW 144
+#define XTX_GM 8
+typedef float xtx_f4 __attribute__((ext_vector_type(4), aligned(4)));   // (X is 4-byte aligned)
+// the tiles above row tile r
+DEV int64_t xtx_before(int64_t r) { return r * (r + 1) / 2; }
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_xtx(
     const float *__restrict__ X, int64_t nrows, int64_t ne0, double *__restrict__ H) {
-    if (blockIdx.y < blockIdx.x) return;                  // (uniform: a tile above the diagonal)
     __shared__ __align__(16) double As[2][XTX_BK][XTX_LDS_ROW];
     __shared__ __align__(16) double Bs[2][XTX_BK][XTX_LDS_ROW];
-    const int64_t row0 = (int64_t)blockIdx.y * 128, col0 = (int64_t)blockIdx.x * 128;
+    const int64_t nr = ne0 / 128, nt = xtx_before(nr), nper = (nt + 7) / 8;
+    const int64_t t = (int64_t)(blockIdx.x % 8) * nper + blockIdx.x / 8;
+    if ((int64_t)(blockIdx.x / 8) >= nper || t >= nt) return;   // (uniform)
+    int64_t g0 = 0;                                       // the group's first row tile
+    while (g0 + XTX_GM < nr && xtx_before(g0 + XTX_GM) <= t) g0 += XTX_GM;
+    const int64_t gm = nr - g0 < XTX_GM ? nr - g0 : XTX_GM, u = t - xtx_before(g0), sq = g0 * gm;
+    int64_t tr, tc;
+    if (u < sq) {                                         // columns that every row of the group has
+        tr = g0 + u % gm;
+        tc = u / gm;
+    } else {                                              // the group's triangle, row by row
+        const int64_t v = u - sq;
+        int64_t r = 0;
+        while (xtx_before(r + 1) <= v) ++r;
+        tr = g0 + r;
+        tc = g0 + (v - xtx_before(r));
+    }
+    const int64_t row0 = tr * 128, col0 = tc * 128;
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     const int wr0 = (wave >> 1) * 64, wc0 = (wave & 1) * 64;
     ldlq_d4 acc[4][4];
@@ -64,25 +90,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b) acc[a][b] = ldlq_d4{0.0, 0.0, 0.0, 0.0};
-    const int lk = tid >> 4, le = tid & 15;                // loader: chunk row lk, elements le + 16 j
-    double av[8], bv[8];
-    auto load = [&](int64_t k0) {
-        const int64_t k = k0 + lk;
-        const bool in = k < nrows;
-        const float *xr = X + (in ? k : 0) * ne0;
+    const int lk = tid >> 4, le = (tid & 15) * 4;          // loader: chunk row lk, elements le + 64 j .. + 3
+    const float *ap = X + row0 + le, *bp = X + col0 + le;
+    xtx_f4 av[2], bv[2];
+    auto load = [&](int64_t k0) {                          // (rows past the end read the last one: stash clears them)
+        const int64_t k = k0 + lk < nrows ? k0 + lk : nrows - 1;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) av[j] = in ? (double)xr[row0 + le + 16 * j] : 0.0;
+        for (int j = 0; j < 2; ++j) av[j] = *(const xtx_f4 *)(ap + k * ne0 + 64 * j);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) bv[j] = in ? (double)xr[col0 + le + 16 * j] : 0.0;
+        for (int j = 0; j < 2; ++j) bv[j] = *(const xtx_f4 *)(bp + k * ne0 + 64 * j);
     };
-    auto stash = [&](int buf) {
+    auto stash = [&](int buf, int64_t k0) {
+        const bool in = k0 + lk < nrows;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) As[buf][lk][le + 16 * j] = av[j];
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) Bs[buf][lk][le + 16 * j] = bv[j];
+            for (int e = 0; e < 4; ++e) As[buf][lk][le + 64 * j + e] = in ? (double)av[j][e] : 0.0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Bs[buf][lk][le + 64 * j + e] = in ? (double)bv[j][e] : 0.0;
     };
     load(0);
-    stash(0);
+    stash(0, 0);
     __syncthreads();
     int buf = 0;
     for (int64_t k0 = 0; k0 < nrows; k0 += XTX_BK) {
@@ -93,32 +123,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             const int kk = ks + lane / 16;
             double a[4], b[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                a[t] = As[buf][kk][wr0 + 16 * t + lane % 16];
-                b[t] = Bs[buf][kk][wc0 + 16 * t + lane % 16];
-            }
+            for (int i = 0; i < 4; ++i) a[i] = As[buf][kk][wr0 + 16 * i + lane % 16];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = Bs[buf][kk][wc0 + 16 * j + lane % 16];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
         }
-        if (more) stash(buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);                 // (the conversions, which wait for the loads, stay here)
+        if (more) stash(buf ^ 1, k0 + XTX_BK);
         __syncthreads();
         buf ^= 1;
     }
     // output element e of lane l: row 4e + l/16, column l%16 of its 16 x 16 tile
+    const bool mirror = tr != tc;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            double *hr = H + (row0 + wr0 + 16 * i + 4 * e + lane / 16) * ne0 + col0 + wc0 + lane % 16;
+        for (int j = 0; j < 4; ++j) {
+            const int64_t r = row0 + wr0 + 16 * i + lane / 16, c = col0 + wc0 + 16 * j + lane % 16;
+            double v[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) hr[16 * j] += acc[i][j][e];
+            for (int e = 0; e < 4; ++e) v[e] = H[(r + 4 * e) * ne0 + c];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) H[(r + 4 * e) * ne0 + c] = v[e] += acc[i][j][e];
+            if (mirror) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) H[c * ne0 + r + 4 * e] = v[e];
+            }
         }
-}
-
-// H[i][j] = H[j][i] for the tiles above the diagonal (i < j and their 128-tiles differ); grid (ceil(ne0 / 256), ne0)
-__global__ __launch_bounds__(256) void k_hess_mirror(double *__restrict__ H, int64_t ne0) {
-    const int64_t i = blockIdx.y, j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (j < ne0 && i / 128 < j / 128) H[i * ne0 + j] = H[j * ne0 + i];
 }
