@@ -629,10 +629,20 @@ bool ldlq_type(int t) {
 
 bool launch_solve(int type, const float *W, const uint8_t *q, int64_t q_stride, int64_t q_off, const double *U,
                   int64_t u_stride, int64_t nmat, int64_t ne1, int64_t ne0, int64_t c0, double *Es, hipStream_t st) {
-    const dim3 grid((unsigned)((ne1 + 63) / 64), (unsigned)nmat);
+    // 16 rows a workgroup while there are at most five for each CU, 64 rows a wave beyond: each workgroup of a CU takes its
+    // 25 us after the one before, the wide kernel 135 us for any number of rows that leaves it a wave a CU (16384) and
+    // 202 us at 57344, where the narrow one takes 349
+    const int64_t groups = (ne1 + LDLQ_SR - 1) / LDLQ_SR;
+    const bool narrow = groups * nmat <= (int64_t)5 * g_ncu;
+    const dim3 grid((unsigned)(narrow ? groups : (ne1 + 63) / 64), (unsigned)nmat);
     const uint64_t *dq = tab_of(type).dq;
-#define KSOLVE(T) hipLaunchKernelGGL((k_ldlq_solve<T>), grid, dim3(64), 0, st, W, q, q_stride, q_off, U, u_stride, \
-                                     ne1, ne0, c0, Es, dq)
+#define KSOLVE(T)                                                                                                         \
+    if (narrow)                                                                                                           \
+        hipLaunchKernelGGL((k_ldlq_solve16<T>), grid, dim3(320), 0, st, W, q, q_stride, q_off, U, u_stride, ne1, ne0, c0, \
+                           Es, dq);                                                                                       \
+    else                                                                                                                  \
+        hipLaunchKernelGGL((k_ldlq_solve<T>), grid, dim3(64), 0, st, W, q, q_stride, q_off, U, u_stride, ne1, ne0, c0,    \
+                           Es, dq)
     switch (type) {
         case T_IQ2_XXS: KSOLVE(T_IQ2_XXS); break;
         case T_IQ2_XS: KSOLVE(T_IQ2_XS); break;

@@ -3,7 +3,7 @@
 // For column block k (256 permuted columns, c0 = 256k) of nmat matrices of ne1 rows:
 //   1. the quantizer runs on the strided view of block k of every row (frame.cuh) and writes each row's block
 //      into its output slot;
-//   2. k_ldlq_solve: E = blk - to_float(block bytes) in f32, then Es = E U_BB^-1 by forward substitution in f64:
+//   2. k_ldlq_solve / k_ldlq_solve16: E = blk - to_float(block bytes) in f32, then Es = E U_BB^-1 by forward substitution in f64:
 //      Es[j] = (E[j] - sum_{i<j} Es[i] U[c0+i][c0+j]) / U[c0+j][c0+j], each sum a fused multiply-add chain over i in
 //      ascending order (the part over earlier 32-column chunks on the matrix cores);
 //   3. k_ldlq_update, an f64 GEMM on the matrix cores: W[r][c] -= (float)(sum_{i<256} Es[r][i] U[c0+i][c]) for the
@@ -26,7 +26,8 @@
 
 typedef double ldlq_d4 __attribute__((ext_vector_type(4)));
 
-// One wave = 64 rows of one matrix (blockIdx.y); the block's 256 columns in chunks of 32. Chunk c:
+// The solve of many rows (fewer go to k_ldlq_solve16, which ends sooner but fills a CU with 16 rows):
+// one wave = 64 rows of one matrix (blockIdx.y); the block's 256 columns in chunks of 32. Chunk c:
 //   E = blk - to_float(bytes) (f32, then f64), one lane a row, into LDS;
 //   E -= Es[:, 0 .. 32c) U[0 .. 32c, chunk] on the f64 matrix cores (each output an fma chain over ascending k,
 //   started from E: the serial loop's order), with Es read back (k-major) from the earlier chunks' stores;
@@ -131,6 +132,214 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         __threadfence_block();
         wave_sync();
     }
+}
+
+// A workgroup of 5 waves owns 16 rows of one matrix (blockIdx.y); E and then Es of the block's 256 columns lie in LDS,
+// column by column. E = blk - to_float(bytes) (f32, then f64) comes from 128 threads, one a row and 32-column chunk. The
+// 16 x 16 MFMA tiles of E, 16 of them, are dealt to four waves in turn and stay in their accumulators. Chunk c:
+//   the two waves that hold its tiles put them into LDS;
+//   the fifth wave solves the 32 x 32 triangle by forward substitution: four lanes a row, each with every fourth column,
+//   the row's next Es passed to the four by DPP, U's diagonal block in LDS;
+//   the four multiply the chunk's Es with U's rows (read while the triangle was solved) into their later tiles, each output
+//   an fma chain over ascending k, started from E: the serial loop's order.
+// The chain of 256 columns bounds it, so a row is spread over lanes and a matrix over workgroups: 4096 rows (IQ2_S) take
+// 25 us, and 135 with k_ldlq_solve, on 64 of the 1024 SIMDs. One workgroup fits a CU (its fifth wave would be the fourth on
+// one of the SIMDs, whose registers hold three), so a GPU-full of rows, 16 a CU, takes another 25 us.
+//
+// x / d, d from U's diagonal: with r = 1 / d correctly rounded (worked out beside the chain), q0 = x r, q1 = q0 + (x - d q0)
+// r and q2 = q1 + (x - d q1) r, each residual one fma: q1 lies within an ulp of x / d, so q2 is the correctly rounded
+// quotient (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990, theorem 8.7
+// of the Handbook of Floating-Point Arithmetic), where no step leaves the normal range: both operands within 2^-500 and
+// 2^500, or x is a zero (q0 is the quotient). A chunk with any other operand is solved over with divisions.
+#define LDLQ_SR 16            // rows a workgroup
+#define LDLQ_TROW 17          // LDS column stride (the tiles' transposed writes spread over the banks)
+#define LDLQ_UROW 34
+// the value of lane S of each four
+template <int S> DEV double quad_bcast(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    constexpr int ctl = S * 0x55;                           // quad_perm [S, S, S, S]
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, ctl, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), ctl, 0xf, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// What column I of the forward substitution reads: lane s of a row's four holds columns 4q + s in x[q]; ud: U's rows,
+// column 4q + s at s * 8 + q; dr: the diagonal and its reciprocal
+struct LdlqRow {
+    double u[8], d, r;
+    template <int I> DEV void load(const double (*ud)[LDLQ_UROW], const double (*dr)[2], int s) {
+#pragma unroll
+        for (int q = I / 4; q < 8; ++q) u[q] = ud[I][s * 8 + q];
+        d = dr[I][0];
+        r = dr[I][1];
+    }
+};
+// the range of the operands: the high word of the largest magnitude, the least exponent (a zero's counts as 0)
+struct LdlqRange {
+    int hi, lo;
+    DEV void see(double v) {
+        hi = imax(hi, (int)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffff);
+        lo = imin(lo, __builtin_amdgcn_frexp_exp(v));
+    }
+    DEV bool mid() const { return hi < (1023 + 500) << 20 && lo > -500; }
+};
+// Columns I .. 31, each row's results to T. Rows of U are read two columns ahead, and no further, and a column's results
+// are worked out in it (the empty asm: left free, the compiler moves the reads up and the later columns' products down, and
+// keeps what lies between in scratch). DIV divides.
+template <int I, bool DIV> DEV void ldlq_columns(double (&x)[8], const LdlqRow &c0, const LdlqRow &c1,
+                                                 const double (*ud)[LDLQ_UROW], const double (*dr)[2], int s,
+                                                 double *out, LdlqRange &rg) {
+    constexpr int Q = I / 4, S = I % 4;
+    LdlqRow c2;
+    if constexpr (I < 30) c2.load<I + 2>(ud, dr, s);
+    const double v = quad_bcast<S>(x[Q]), d = c0.d;
+    double xi;
+    if (DIV) {
+        xi = v / d;
+    } else {
+        const double r = c0.r, q0 = v * r, q1 = fma(fma(-d, q0, v), r, q0);
+        xi = __builtin_copysign(fma(fma(-d, q1, v), r, q1), q0);         // (a zero's sign is q0's)
+        rg.see(v);
+    }
+    out[I * LDLQ_TROW] = xi;                                // (the four lanes write the same value)
+#pragma unroll
+    for (int q = Q; q < 8; ++q) x[q] = fma(-xi, c0.u[q], x[q]);          // (columns up to I are not read again)
+#pragma unroll
+    for (int q = Q; q < 8; ++q) asm volatile("" : "+v"(x[q]));
+    asm volatile("" : "+v"(rg.hi), "+v"(rg.lo) :: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (I < 31) ldlq_columns<I + 1, DIV>(x, c1, c2, ud, dr, s, out, rg);
+}
+// one chunk's triangle, x to be overwritten; false: an operand was out of the short division's range
+template <bool DIV> DEV bool ldlq_triangle(double (&x)[8], const double (*ud)[LDLQ_UROW], const double (*dr)[2], int s,
+                                           double *out) {
+    LdlqRange rg{0, 0};
+    if (!DIV) {
+        const double d = dr[lane_id() & 31][0];
+        rg.see(d);
+        rg.lo = d == 0.0 ? -1000 : rg.lo;
+    }
+    LdlqRow c0, c1;
+    c0.load<0>(ud, dr, s);
+    c1.load<1>(ud, dr, s);
+    ldlq_columns<0, DIV>(x, c0, c1, ud, dr, s, out, rg);
+    return DIV || rg.mid();
+}
+
+template <int TYPE>
+__global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(3))) void k_ldlq_solve16(
+    const float *__restrict__ W, const uint8_t *__restrict__ q, int64_t q_stride, int64_t q_off,
+    const double *__restrict__ U, int64_t u_stride, int64_t ne1, int64_t ne0, int64_t c0, double *__restrict__ Es,
+    const uint64_t *__restrict__ grid) {
+    __shared__ double T[QK][LDLQ_TROW];                     // E, then Es: [column][row]
+    __shared__ __align__(16) double Ud[2][32][LDLQ_UROW];                // U's diagonal block of the chunk, of the next one
+    __shared__ __align__(16) double Dr[2][32][2];           // and its diagonal, with the reciprocals
+    const int64_t m = blockIdx.y, row0 = (int64_t)blockIdx.x * LDLQ_SR;
+    const int tid = threadIdx.x, lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t R = (int64_t)gridDim.y * ne1;             // Es rows (k-major: Es[k * R + r])
+    const double *Ub = U + m * u_stride + c0 * ne0 + c0;    // the block's diagonal square
+    double du[4], dd = 1.0;
+    auto load_diag = [&](int c) {
+        const double *p = Ub + (int64_t)(32 * c) * ne0 + 32 * c;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) du[j] = p[(int64_t)((tid >> 5) + 8 * j) * ne0 + (tid & 31)];
+        if (tid < 32) dd = p[(int64_t)tid * ne0 + tid];
+    };
+    auto stash_diag = [&](int c) {
+        const int t = tid & 31;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) Ud[c & 1][(tid >> 5) + 8 * j][(t & 3) * 8 + (t >> 2)] = du[j];
+        if (tid < 32) {
+            Dr[c & 1][tid][0] = dd;
+            Dr[c & 1][tid][1] = 1.0 / dd;
+        }
+    };
+    if (wave < 4) load_diag(0);
+    if (tid < 128) {
+        const int r = tid & 15, c = tid >> 4;
+        // (rows past the matrix read row ne1 - 1: their results are not stored)
+        const int64_t gr = m * ne1 + (row0 + r < ne1 ? row0 + r : ne1 - 1);
+        const float4 *wp = (const float4 *)(W + gr * ne0 + c0 + 32 * c);
+        float y[32];
+        dq_chunk<TYPE>(q + gr * q_stride + q_off, c, y, grid);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const float4 v = wp[t];
+            T[32 * c + 4 * t + 0][r] = (double)(v.x - y[4 * t + 0]);
+            T[32 * c + 4 * t + 1][r] = (double)(v.y - y[4 * t + 1]);
+            T[32 * c + 4 * t + 2][r] = (double)(v.z - y[4 * t + 2]);
+            T[32 * c + 4 * t + 3][r] = (double)(v.w - y[4 * t + 3]);
+        }
+    }
+    if (wave < 4) stash_diag(0);
+    __syncthreads();
+    const int lx = lane & 15, ly = lane >> 4;
+    if (wave == 4) {                                        // the triangles
+        const int r = lane >> 2, s = lane & 3;
+#pragma unroll 1
+        for (int c = 0; c < 8; ++c) {
+            __syncthreads();
+            double x[8], x0[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = x0[i] = T[32 * c + 4 * i + s][r];
+            const bool ok = ldlq_triangle<false>(x, Ud[c & 1], Dr[c & 1], s, &T[32 * c][r]);
+            if (__ballot(!ok)) ldlq_triangle<true>(x0, Ud[c & 1], Dr[c & 1], s, &T[32 * c][r]);
+            __syncthreads();
+        }
+        return;
+    }
+    ldlq_d4 acc[4];                                         // tiles wave, wave + 4, wave + 8, wave + 12
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[u][e] = T[16 * (wave + 4 * u) + lx][4 * e + ly];
+    // chunks 2h and 2h + 1: of the wave's tiles, number h is in one of them, and those after it are still to come
+    auto half = [&](auto hc) {
+        constexpr int h = decltype(hc)::value;
+#pragma unroll 1
+        for (int c = 2 * h; c < 2 * h + 2; ++c) {
+            const bool own = (wave >> 1) == (c & 1), mine = (wave >> 1) > (c & 1);   // tile h is in the chunk / after it
+            if (c > 0 && own) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) T[16 * (wave + 4 * h) + lx][4 * e + ly] = acc[h][e];
+            }
+            __syncthreads();
+            // the triangle is solved meanwhile
+            const double *Uc = Ub + (int64_t)(32 * c + ly) * ne0 + 16 * wave + lx;
+            double b[4][8];
+            if (mine)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) b[h][k] = Uc[(int64_t)(4 * k) * ne0 + 64 * h];
+#pragma unroll
+            for (int u = h + 1; u < 4; ++u)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) b[u][k] = Uc[(int64_t)(4 * k) * ne0 + 64 * u];
+            if (c < 7) {
+                load_diag(c + 1);
+                stash_diag(c + 1);                          // (the other buffer: last read before the last barrier)
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int k = 32 * c + (tid >> 4) + 16 * j, r = tid & 15;
+                if (row0 + r < ne1) Es[k * R + m * ne1 + row0 + r] = T[k][r];
+            }
+            double a[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) a[k] = -T[32 * c + 4 * k + ly][lx];
+            if (mine)                                       // (the next chunk's tiles first: the triangle waits for them)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], b[h][k], acc[h], 0, 0, 0);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+#pragma unroll
+                for (int u = h + 1; u < 4; ++u)
+                    acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], b[u][k], acc[u], 0, 0, 0);
+        }
+    };
+    half(std::integral_constant<int, 0>{});
+    half(std::integral_constant<int, 1>{});
+    half(std::integral_constant<int, 2>{});
+    half(std::integral_constant<int, 3>{});
 }
 
 // W[m][row][c] -= (float)(sum_i Es[c0+i][m*ne1+row] U_m[c0+i][c]) for c in [cb, ce) (later columns than block
