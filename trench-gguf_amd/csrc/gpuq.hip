@@ -614,9 +614,15 @@ bool side_stream_ready() {
 // W -= Es . U[c0 .. c0+255][cb .. ce) for every matrix
 bool launch_update(float *W, const double *Es, const double *U, int64_t u_stride, int64_t nmat, int64_t ne1,
                    int64_t ne0, int64_t c0, int64_t cb, int64_t ce, hipStream_t st) {
-    const int64_t nt = ((ce - cb + LDLQ_TN - 1) / LDLQ_TN) * ((ne1 + LDLQ_TM - 1) / LDLQ_TM) * nmat;
-    const unsigned grid = (unsigned)((nt + 7) / 8 * 8);   // (a multiple of the 8 XCDs; see ldlq_tile)
-    hipLaunchKernelGGL(k_ldlq_update, dim3(grid), dim3(256), 0, st, W, Es, U, u_stride, nmat, ne1, ne0, c0, cb, ce);
+    auto tiles = [&](int64_t t) { return ((ce - cb + t - 1) / t) * ((ne1 + t - 1) / t) * nmat; };
+    // 128 x 128 tiles, or 64 x 64 where those would leave CUs without one: the next block's 256 columns of fewer than
+    // 16384 rows, which the loop waits for (4096 rows, 64 tiles: 42 us; 256 of the others: 19 us), and the last blocks' rest
+    const bool small = tiles(128) < g_ncu;
+    const unsigned grid = (unsigned)((tiles(small ? 64 : 128) + 7) / 8 * 8);   // (a multiple of the 8 XCDs; see ldlq_tile)
+    if (small)
+        hipLaunchKernelGGL(k_ldlq_update<64>, dim3(grid), dim3(256), 0, st, W, Es, U, u_stride, nmat, ne1, ne0, c0, cb, ce);
+    else
+        hipLaunchKernelGGL(k_ldlq_update<128>, dim3(grid), dim3(256), 0, st, W, Es, U, u_stride, nmat, ne1, ne0, c0, cb, ce);
     return hipGetLastError() == hipSuccess;
 }
 

@@ -21,8 +21,6 @@
 #ifndef LDLQ_BK
 #define LDLQ_BK 16            // k-chunk of the update GEMM
 #endif
-#define LDLQ_TM 128           // update tile rows
-#define LDLQ_TN 128           // update tile columns
 
 typedef double ldlq_d4 __attribute__((ext_vector_type(4)));
 
@@ -343,17 +341,16 @@ __global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(3))) void k
 }
 
 // W[m][row][c] -= (float)(sum_i Es[c0+i][m*ne1+row] U_m[c0+i][c]) for c in [cb, ce) (later columns than block
-// c0's: cb >= c0 + 256). Es is k-major (Es[k][row], k < 256). A workgroup of 4 waves owns a 128 x 128 tile (each
-// wave 64 x 64: 4 x 4 MFMA tiles of 16 x 16); k runs in chunks of 16 staged in LDS, k-major, two buffers (one barrier
+// c0's: cb >= c0 + 256). Es is k-major (Es[k][row], k < 256). A workgroup of 4 waves owns a TT x TT tile, 128
+// or 64 a side (each wave a quarter: 4 x 4 or 2 x 2 MFMA tiles of 16 x 16; launch_update chooses); k runs in chunks of 16 staged in LDS, k-major, two buffers (one barrier
 // a chunk). A loader thread moves k row t/16, elements t%16 + 16j: 16 lanes read 128 contiguous bytes and write 16
-// consecutive LDS doubles; LDS rows are 144 doubles apart (1152 B = 128 mod 256), so the MFMA operand reads (4 k
+// consecutive LDS doubles; LDS rows are TT + 16 doubles apart (128 B mod 256), so the MFMA operand reads (4 k
 // rows x 16 consecutive doubles a wave) and the loader's writes fall in distinct banks.
 //
 // Tiles are numbered matrix by matrix, and within a matrix in groups of LDLQ_GM row tiles, rows fastest, so that the
 // workgroups running together share LDLQ_GM Es panels and as many U panels. The 1-D grid (padded to a multiple of
 // 8) is dealt to the 8 XCDs round-robin, so workgroup i takes tile (i % 8) * nper + i / 8: each XCD works through one
-// contiguous range of tiles and its L2 holds the panels they share (128 x 256 doubles each, 256 KB).
-#define LDLQ_LDS_ROW 144
+// contiguous range of tiles and its L2 holds the panels they share (128 x 256 doubles each, 256 KB; half that for TT 64).
 #define LDLQ_GM 8
 DEV bool ldlq_tile(int64_t ntr, int64_t ntc, int64_t nmat, int64_t &m, int64_t &tr, int64_t &tc) {
     const int64_t nt = ntr * ntc * nmat, nper = (nt + 7) / 8;
@@ -368,53 +365,55 @@ DEV bool ldlq_tile(int64_t ntr, int64_t ntc, int64_t nmat, int64_t &m, int64_t &
     tc = v / gm;
     return true;
 }
+template <int TT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_ldlq_update(
     float *__restrict__ W, const double *__restrict__ Es, const double *__restrict__ U, int64_t u_stride, int64_t nmat,
     int64_t ne1, int64_t ne0, int64_t c0, int64_t cb, int64_t ce) {
-    __shared__ __align__(16) double As[2][LDLQ_BK][LDLQ_LDS_ROW];
-    __shared__ __align__(16) double Bs[2][LDLQ_BK][LDLQ_LDS_ROW];
+    __shared__ __align__(16) double As[2][LDLQ_BK][TT + 16];
+    __shared__ __align__(16) double Bs[2][LDLQ_BK][TT + 16];
     int64_t m, tr, tc;
-    if (!ldlq_tile((ne1 + LDLQ_TM - 1) / LDLQ_TM, (ce - cb + LDLQ_TN - 1) / LDLQ_TN, nmat, m, tr, tc)) return;
+    if (!ldlq_tile((ne1 + TT - 1) / TT, (ce - cb + TT - 1) / TT, nmat, m, tr, tc)) return;
     const int64_t R = nmat * ne1;
-    const int64_t row0 = tr * LDLQ_TM;
-    const int64_t col0 = cb + tc * LDLQ_TN;
+    const int64_t row0 = tr * TT;
+    const int64_t col0 = cb + tc * TT;
     const double *Um = U + m * u_stride;
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
-    const int wr0 = (wave >> 1) * 64, wc0 = (wave & 1) * 64;   // the wave's 64 x 64 sub-tile
-    ldlq_d4 acc[4][4];
+    constexpr int NT = TT / 32, NL = TT / 16;                  // 16 x 16 tiles a side of the wave's sub-tile; loads
+    const int wr0 = (wave >> 1) * (TT / 2), wc0 = (wave & 1) * (TT / 2);
+    ldlq_d4 acc[NT][NT];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NT; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = ldlq_d4{0.0, 0.0, 0.0, 0.0};
-    static_assert(LDLQ_BK * 16 == 256 && LDLQ_TM == 128 && LDLQ_TN == 128, "loader: 16 k rows x 16 lanes, 8 a thread");
+        for (int b = 0; b < NT; ++b) acc[a][b] = ldlq_d4{0.0, 0.0, 0.0, 0.0};
+    static_assert(LDLQ_BK * 16 == 256 && (TT == 128 || TT == 64), "loader: 16 k rows x 16 lanes, NL a thread");
     const int lk = tid >> 4, le = tid & 15;
     const double *abase = Es + m * ne1 + row0 + le;          // + k * R + 16 j
     const double *bbase = Um + col0 + le;                     // + (c0 + k) * ne0 + 16 j
-    double av[8], bv[8];
+    double av[NL], bv[NL];
     // a tile inside the matrix (the usual case) loads unguarded: no per-element branches
-    const bool full = row0 + LDLQ_TM <= ne1 && col0 + LDLQ_TN <= ce;
+    const bool full = row0 + TT <= ne1 && col0 + TT <= ce;
     auto load = [&](int k0) {
         const double *ap = abase + (int64_t)(k0 + lk) * R;
         const double *bp = bbase + (c0 + k0 + lk) * ne0;
         if (full) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) av[j] = ap[16 * j];
+            for (int j = 0; j < NL; ++j) av[j] = ap[16 * j];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bv[j] = bp[16 * j];
+            for (int j = 0; j < NL; ++j) bv[j] = bp[16 * j];
         } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) av[j] = row0 + le + 16 * j < ne1 ? ap[16 * j] : 0.0;
+            for (int j = 0; j < NL; ++j) av[j] = row0 + le + 16 * j < ne1 ? ap[16 * j] : 0.0;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bv[j] = col0 + le + 16 * j < ce ? bp[16 * j] : 0.0;
+            for (int j = 0; j < NL; ++j) bv[j] = col0 + le + 16 * j < ce ? bp[16 * j] : 0.0;
         }
     };
     auto stash = [&](int buf) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) As[buf][lk][le + 16 * j] = av[j];
+        for (int j = 0; j < NL; ++j) As[buf][lk][le + 16 * j] = av[j];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) Bs[buf][lk][le + 16 * j] = bv[j];
+        for (int j = 0; j < NL; ++j) Bs[buf][lk][le + 16 * j] = bv[j];
     };
-    float wv[4][4][4];                      // the wave's W values (full tiles: read during the last chunk)
+    float wv[NT][4][NT];                      // the wave's W values (full tiles: read during the last chunk)
     auto read_w = [&](int i0, int i1) {
 #pragma unroll
         for (int i = i0; i < i1; ++i)
@@ -422,23 +421,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             for (int e = 0; e < 4; ++e) {
                 const float *wr = W + (m * ne1 + row0 + wr0 + 16 * i + 4 * e + lane / 16) * ne0 + col0 + wc0 + lane % 16;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) wv[i][e][j] = wr[16 * j];
+                for (int j = 0; j < NT; ++j) wv[i][e][j] = wr[16 * j];
             }
     };
     auto chunk = [&](int buf) {             // this wave's MFMAs over the staged k-chunk
 #pragma unroll
         for (int ks = 0; ks < LDLQ_BK; ks += 4) {
             const int kk = ks + lane / 16;
-            double a[4], b[4];
+            double a[NT], b[NT];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < NT; ++t) {
                 a[t] = As[buf][kk][wr0 + 16 * t + lane % 16];
                 b[t] = Bs[buf][kk][wc0 + 16 * t + lane % 16];
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < NT; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
         }
     };
     load(0);
@@ -454,42 +453,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
     if (full) read_w(0, 1);                 // half the epilogue's reads overlap the last chunk's MFMAs (all of
     chunk(buf);                             // them would not fit in the registers beside the accumulators)
-    if (full) read_w(1, 4);
+    if (full) read_w(1, NT);
     // epilogue: every W value of the wave's sub-tile is read before the first store (a store between the reads
     // would make each read wait for the one before it); a full tile runs unguarded, so the stores need no
     // per-element branches (and their waits no conservative counts)
     if (full) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NT; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float *wr = W + (m * ne1 + row0 + wr0 + 16 * i + 4 * e + lane / 16) * ne0 + col0 + wc0 + lane % 16;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) wr[16 * j] = wv[i][e][j] - (float)acc[i][j][e];
+                for (int j = 0; j < NT; ++j) wr[16 * j] = wv[i][e][j] - (float)acc[i][j][e];
             }
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int64_t row = row0 + wr0 + 16 * i + 4 * e + lane / 16;
             const float *wr = W + (m * ne1 + (row < ne1 ? row : 0)) * ne0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < NT; ++j) {
                 const int64_t col = col0 + wc0 + 16 * j + lane % 16;
                 wv[i][e][j] = row < ne1 && col < ce ? wr[col] : 0.f;
             }
         }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int64_t row = row0 + wr0 + 16 * i + 4 * e + lane / 16;
             if (row >= ne1) continue;
             float *wr = W + (m * ne1 + row) * ne0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < NT; ++j) {
                 const int64_t col = col0 + wc0 + 16 * j + lane % 16;
                 if (col < ce) wr[col] = wv[i][e][j] - (float)acc[i][j][e];
             }
