@@ -7,8 +7,8 @@
 // order-free reductions (max). A wave therefore quantizes 64/G super-blocks at once, with 100% lane occupancy in the
 // fixed-trip-count search loops. Each wave assembles its super-blocks' output bytes in an LDS image and writes them
 // to HBM as one contiguous, dword-coalesced range. For the types with neighbour searches (tiles of varying cost) the
-// launch holds as many workgroups as the CUs keep resident, and each wave takes its tiles (64/G super-blocks) one at
-// a time from a counter: the waves sweep the tensor once, in order (an expert's importance row is read while the
+// launch holds as many workgroups as the CUs keep resident, and each wave takes its tiles (64/G super-blocks, fewer in
+// calls that would leave waves without one) one at a time from a counter, unless each has its only one from the start: the waves sweep the tensor once, in order (an expert's importance row is read while the
 // whole chip works on that expert), every wave busy until the counter runs past the end. The other types loop over
 // the tiles grid-stride. The per-workgroup LDS table staging of the i-quants is paid once per workgroup.
 #pragma once
@@ -37,6 +37,7 @@ struct QParams {
     // number) each wave takes the next from it (grid waves + the counter's old value), so the resident waves sweep
     // the tensor once, in order, and finish together; nullptr: a fixed grid-stride order
     unsigned long long *tiles;
+    int spw;                // queue types: units a tile (64/G, or 2 or more of them in calls of few units: launch_q)
     // strided views (the LDLQ loop quantizes one block column of every row): unit b reads its weights at element
     // b*sb_stride + sb_off, its importance at row*qw_stride + qw_off, and writes its block at byte
     // b*out_stride + out_off. The contiguous defaults are sb_stride = BS, qw_stride = BS, out_stride = BB, 0 offsets.
@@ -144,6 +145,9 @@ template <class T> struct wgw_of<T, decltype((void)T::WGW)> { static constexpr i
 // resident grid; without it a grid-stride order over up to 32 waves a CU (tiles of equal cost)
 template <class T, class = void> struct queue_of { static constexpr bool v = false; };
 template <class T> struct queue_of<T, decltype((void)T::QUEUE)> { static constexpr bool v = T::QUEUE; };
+// THIN (optional, false): a queue type that keeps whole tiles in calls of few units (launch_q)
+template <class T, class = void> struct thin_of { static constexpr bool v = queue_of<T>::v; };
+template <class T> struct thin_of<T, decltype((void)T::THIN)> { static constexpr bool v = T::THIN; };
 // ROWSIG (optional): quant_rs takes the unit's row-wide sigma2 (p.rsig) after its importance row
 template <class T, class = void> struct rowsig_of { static constexpr bool v = false; };
 template <class T> struct rowsig_of<T, decltype((void)T::ROWSIG)> { static constexpr bool v = T::ROWSIG; };
@@ -155,7 +159,7 @@ template <class T, int SRC>
 __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_eu(wpe_of<T>::v))) void k_quant(
     QParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int SPW = 64 / T::G, WGW = wgw_of<T>::v;
+    constexpr int SPW = 64 / T::G;
     if (T::TAB) {
         T::stage(p, lds);
         __syncthreads();
@@ -163,24 +167,30 @@ __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_
     const int wave = (int)(threadIdx.x >> 6), lane = lane_id();
     const int g = lane % T::G, slot = lane / T::G;
     uint8_t *img = lds + T::TAB + wave * wave_bytes<T>();
-    const int64_t nwaves = (int64_t)gridDim.x * WGW;
+    const int wgw = thin_of<T>::v ? (int)(blockDim.x >> 6) : wgw_of<T>::v, spw = thin_of<T>::v ? p.spw : SPW;
+    const int64_t nwaves = (int64_t)gridDim.x * wgw;
     const bool queue = queue_of<T>::v && p.tiles != nullptr;       // (compile-time false for the other types)
     // queued tiles come in chunks of KT whose source bytes start and end on 128-byte lines (the 17-byte MXFP4 and
     // 34-byte Q8_0 blocks), so that no line is fetched by two waves of different XCDs
     constexpr int KT = !queue_of<T>::v ? 1 : SRC == T_MXFP4 ? (SPW >= 16 ? 1 : 16 / SPW)
                                            : SRC == T_Q8_0 ? (SPW >= 8 ? 1 : 8 / SPW) : 1;
-    int64_t c = (int64_t)blockIdx.x * WGW + wave;        // (the first chunks in wave order: no burst on the counter)
+    const int kt = !thin_of<T>::v || spw == SPW ? KT : 1;
+    int64_t c = (int64_t)blockIdx.x * wgw + wave;        // (the first chunks in wave order: no burst on the counter)
     int k = 0;                                           // the tile in the chunk
-    int64_t t = c * KT;
+    int64_t t = c * kt;
     unsigned long long tn = 0;
-    while (t * SPW < p.nsb) {
-        const int64_t b0 = t * SPW;
-        const int nact = (int)(p.nsb - b0 < SPW ? p.nsb - b0 : SPW);
+    while (t * spw < p.nsb) {
+        const int64_t b0 = t * spw;
+        const int nact = (int)(p.nsb - b0 < spw ? p.nsb - b0 : spw);
         const int64_t b = b0 + (slot < nact ? slot : nact - 1);
         img_zero(img, img_bytes<T>());
         wave_sync();
         float x[T::N];
         SrcLoad<SRC, T::N>::load(p.src, b * p.sb_stride + p.sb_off + g * T::N, x);
+        if (thin_of<T>::v && slot >= nact) {           // a lane without a unit: zeros, which search nothing
+#pragma unroll
+            for (int i = 0; i < T::N; ++i) x[i] = 0.f;
+        }
         // the next chunk, asked for at a chunk's first tile (lane 0's atomic returns while the chunk is quantized)
         if (queue && k == 0 && lane == 0) tn = atomicAdd(p.tiles, 1ull);
         const float *qw = p.qw ? p.qw + qw_row(p, b) * p.qw_stride + p.qw_off + g * T::N : nullptr;
@@ -197,10 +207,10 @@ __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_
             for (int h = g; h < T::BB / 2; h += T::G) o[h] = s[h];
         }
         wave_sync();
-        if (++k == KT) {
+        if (++k == kt) {
             c = queue ? nwaves + wave_u64(tn) : c + nwaves;
             k = 0;
         }
-        t = c * KT + k;
+        t = c * kt + k;
     }
 }

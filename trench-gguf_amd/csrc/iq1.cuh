@@ -163,6 +163,7 @@ template <int G, int N> DEV void grp_chain_sum2(const float (&a)[N], const float
 // block: d qs[32] qh[8] u16 (50 bytes); lane g = 32-weight block g
 struct KIQ1S : Iq8Tab<2048> {
     static constexpr int BS = QK, G = 8, N = 32, BB = 50, WS = coop_wsm_bytes<2, 16, true>(), WGW = 8;
+    static constexpr bool THIN = false;
     static constexpr bool QUEUE = true;         // (tiles of varying cost: the tile queue)
     static DEV void quant(const float (&x)[N], const float *qwp, int g, uint8_t *img, int boff, uint8_t *lds,
                           const QParams &p) {
@@ -371,6 +372,7 @@ DEV void iq1m_sums(float a0x, float a1x, float a0w, float a1w, float b0x, float 
 // block: qs[32] qh[16] scales[8] (56 bytes); lane g = 16-weight block g
 struct KIQ1M : Iq8Tab<2048> {
     static constexpr int BS = QK, G = 16, N = 16, BB = 56, WS = coop_wsm_bytes<2, 16, true>(), WGW = 8;
+    static constexpr bool THIN = false;
     static constexpr bool QUEUE = true;         // (tiles of varying cost: the tile queue)
     static DEV void quant(const float (&x)[N], const float *qwp, int g, uint8_t *img, int boff, uint8_t *lds,
                           const QParams &p) {
