@@ -37,7 +37,6 @@ struct QParams {
     // number) each wave takes the next from it (grid waves + the counter's old value), so the resident waves sweep
     // the tensor once, in order, and finish together; nullptr: a fixed grid-stride order
     unsigned long long *tiles;
-    int spw;                // queue types: units a tile (64/G, or 2 or more of them in calls of few units: launch_q)
     // strided views (the LDLQ loop quantizes one block column of every row): unit b reads its weights at element
     // b*sb_stride + sb_off, its importance at row*qw_stride + qw_off, and writes its block at byte
     // b*out_stride + out_off. The contiguous defaults are sb_stride = BS, qw_stride = BS, out_stride = BB, 0 offsets.
@@ -45,6 +44,7 @@ struct QParams {
     // the row-wide sigma2 of the Q4_0 / Q5_0 / Q5_1 imatrix rules (one a row: unit b is in row b / row_units)
     const float *rsig;
     int64_t row_units;
+    int spw;                // thin tiles: units a tile (launch_q)
 };
 
 // map3 entries: >= 0 a grid index; < 0 an off-grid key, -1 - (list offset | list length << M3_OFF_BITS)
@@ -155,7 +155,10 @@ template <class T> struct rowsig_of<T, decltype((void)T::ROWSIG)> { static const
 template <class T, class = void> struct wpe_of { static constexpr int v = 2; };
 template <class T> struct wpe_of<T, decltype((void)T::WPE)> { static constexpr int v = T::WPE; };
 
-template <class T, int SRC>
+// TH (thin tiles): a call of few units, p.spw of them a tile, one tile a wave and as many waves a workgroup as launched.
+// Kernels of their own, so that large calls run with constants: with the tile's size read at run time 229,376 super-blocks
+// took 3463 us (IQ3_XXS from BF16) and 1444 (IQ2_S from Q8_0), without 3387 and 1420.
+template <class T, int SRC, bool TH>
 __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_eu(wpe_of<T>::v))) void k_quant(
     QParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -167,14 +170,14 @@ __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_
     const int wave = (int)(threadIdx.x >> 6), lane = lane_id();
     const int g = lane % T::G, slot = lane / T::G;
     uint8_t *img = lds + T::TAB + wave * wave_bytes<T>();
-    const int wgw = thin_of<T>::v ? (int)(blockDim.x >> 6) : wgw_of<T>::v, spw = thin_of<T>::v ? p.spw : SPW;
+    const int wgw = TH ? (int)(blockDim.x >> 6) : wgw_of<T>::v, spw = TH ? p.spw : SPW;
     const int64_t nwaves = (int64_t)gridDim.x * wgw;
-    const bool queue = queue_of<T>::v && p.tiles != nullptr;       // (compile-time false for the other types)
+    const bool queue = !TH && queue_of<T>::v && p.tiles != nullptr;       // (compile-time false for the other types)
     // queued tiles come in chunks of KT whose source bytes start and end on 128-byte lines (the 17-byte MXFP4 and
     // 34-byte Q8_0 blocks), so that no line is fetched by two waves of different XCDs
     constexpr int KT = !queue_of<T>::v ? 1 : SRC == T_MXFP4 ? (SPW >= 16 ? 1 : 16 / SPW)
                                            : SRC == T_Q8_0 ? (SPW >= 8 ? 1 : 8 / SPW) : 1;
-    const int kt = !thin_of<T>::v || spw == SPW ? KT : 1;
+    constexpr int kt = TH ? 1 : KT;
     int64_t c = (int64_t)blockIdx.x * wgw + wave;        // (the first chunks in wave order: no burst on the counter)
     int k = 0;                                           // the tile in the chunk
     int64_t t = c * kt;
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_
         wave_sync();
         float x[T::N];
         SrcLoad<SRC, T::N>::load(p.src, b * p.sb_stride + p.sb_off + g * T::N, x);
-        if (thin_of<T>::v && slot >= nact) {           // a lane without a unit: zeros, which search nothing
+        if (TH && slot >= nact) {           // a lane without a unit: zeros, which search nothing
 #pragma unroll
             for (int i = 0; i < T::N; ++i) x[i] = 0.f;
         }
@@ -207,6 +210,7 @@ __global__ __launch_bounds__(64 * wgw_of<T>::v) __attribute__((amdgpu_waves_per_
             for (int h = g; h < T::BB / 2; h += T::G) o[h] = s[h];
         }
         wave_sync();
+        if (TH) break;                                   // (its only tile)
         if (++k == kt) {
             c = queue ? nwaves + wave_u64(tn) : c + nwaves;
             k = 0;

@@ -209,8 +209,9 @@ template <class V> bool upload(V **dst, const std::vector<V> &src) {
 // once: a wave's searches are dealt to all its lanes, so a tile of fewer units ends sooner. 1024 super-blocks, microseconds:
 // IQ2_XXS 135 -> 96, IQ2_XS 80 -> 62, IQ2_S 59 -> 49, IQ3_XXS 267 -> 167, IQ3_S 193 -> 116;
 // 8192: IQ3_XXS 276 -> 216, IQ3_S 200 -> 155, the others equal or a little better. Not below two units: one alone gives 3 to
-// 7% more, but IQ2_XXS takes 113. IQ1_S and IQ1_M keep whole tiles: IQ1_M's kernel is 20% slower on large calls (5.34 ->
-// 6.39 ms on 16 experts) when the tile's size is not a constant.
+// 7% more, but IQ2_XXS takes 113. Thin tiles have kernels of their own (k_quant's TH); IQ1_S and IQ1_M have none: they were
+// measured only with the size read at run time in the one kernel, which cost IQ1_M's large calls 20% (5.34 -> 6.39 ms on 16
+// experts).
 template <class T, int SRC> bool launch_q(const QParams &p0, hipStream_t st) {
     constexpr int SPW = 64 / T::G, WGW = wgw_of<T>::v;
     static_assert((size_t)T::TAB + WGW * wave_bytes<T>() <= 160 * 1024, "a workgroup's LDS within a CU's 160 KiB");
@@ -221,24 +222,32 @@ template <class T, int SRC> bool launch_q(const QParams &p0, hipStream_t st) {
     p.spw = SPW;
     if (!queue_of<T>::v || g_device < 0 || g_device >= 64 || !g_tile_ctr[g_device]) {
         const int64_t wgs = std::max<int64_t>(1, std::min(cap, ((p.nsb + SPW - 1) / SPW + WGW - 1) / WGW));
-        hipLaunchKernelGGL((k_quant<T, SRC>), dim3((unsigned)wgs), dim3(64 * WGW), lds, st, p);
+        hipLaunchKernelGGL((k_quant<T, SRC, false>), dim3((unsigned)wgs), dim3(64 * WGW), lds, st, p);
         return hipGetLastError() == hipSuccess;
     }
     static std::atomic<int> occ{0};
     int n = occ.load();
     if (n == 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_quant<T, SRC>, 64 * WGW, lds) != hipSuccess || n < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_quant<T, SRC, false>, 64 * WGW, lds) != hipSuccess || n < 1)
             return false;
         occ.store(n);
     }
     const int64_t resident = (int64_t)g_ncu * n * WGW;
-    while (thin_of<T>::v && p.spw > 2 && (p.nsb + p.spw / 2 - 1) / (p.spw / 2) <= resident) p.spw /= 2;
-    const int64_t tiles = (p.nsb + p.spw - 1) / p.spw;
-    // thin tiles: workgroups of four waves (one a SIMD) while the CUs have room for them
-    const int wgw = p.spw < SPW && tiles <= (int64_t)g_ncu * 4 ? std::min(4, WGW) : WGW;
-    int64_t wgs = std::min((tiles + wgw - 1) / wgw, (int64_t)g_ncu * n * WGW / wgw);
-    wgs = std::max<int64_t>(wgs, 1);
-    if (wgs * wgw < tiles) {        // (else every wave has its tile from the start)
+    if constexpr (thin_of<T>::v) {
+        while (p.spw > 2 && (p.nsb + p.spw / 2 - 1) / (p.spw / 2) <= resident) p.spw /= 2;
+        if (p.spw < SPW) {
+            const int64_t tiles = (p.nsb + p.spw - 1) / p.spw;
+            // workgroups of four waves (one a SIMD) while the CUs have room for them
+            const int wgw = tiles <= (int64_t)g_ncu * 4 ? std::min(4, WGW) : WGW;
+            const int64_t wgs = std::max<int64_t>(1, (tiles + wgw - 1) / wgw);
+            hipLaunchKernelGGL((k_quant<T, SRC, true>), dim3((unsigned)wgs), dim3(64 * wgw),
+                               (size_t)T::TAB + wgw * wave_bytes<T>(), st, p);
+            return hipGetLastError() == hipSuccess;
+        }
+    }
+    const int64_t tiles = (p.nsb + SPW - 1) / SPW;
+    const int64_t wgs = std::max<int64_t>(1, std::min((tiles + WGW - 1) / WGW, (int64_t)g_ncu * n));
+    if (wgs * WGW < tiles) {        // (else no wave takes a second chunk)
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(st, &cs) != hipSuccess) return false;
         unsigned slot;
@@ -257,7 +266,7 @@ template <class T, int SRC> bool launch_q(const QParams &p0, hipStream_t st) {
         p.tiles = g_tile_ctr[g_device] + slot;
         hipLaunchKernelGGL(k_tile_reset, dim3(1), dim3(64), 0, st, p.tiles);
     }
-    hipLaunchKernelGGL((k_quant<T, SRC>), dim3((unsigned)wgs), dim3(64 * wgw), (size_t)T::TAB + wgw * wave_bytes<T>(), st, p);
+    hipLaunchKernelGGL((k_quant<T, SRC, false>), dim3((unsigned)wgs), dim3(64 * WGW), lds, st, p);
     return hipGetLastError() == hipSuccess;
 }
 
