@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 Q4_0, BF16, F32 = 2, 30, 0
 
 
-def run(oracle_lib, src, nrow, ncol, same_as=None):
+def run(oracle_lib, src, nrow, ncol):
     import torch
     torch.cuda.init()
     import gpuq
@@ -29,7 +29,10 @@ def run(oracle_lib, src, nrow, ncol, same_as=None):
     assert gq.gpuq_requantize_dev(src, d_raw.data_ptr(), Q4_0, out.data_ptr(), 1, nrow, ncol, d_im.data_ptr(),
                                   torch.cuda.current_stream().cuda_stream) == out.numel()
     torch.cuda.synchronize()
-    assert np.array_equal(out.cpu().numpy(), oracle_lib.quantize(Q4_0, x, im).reshape(-1))
+    # (rows stand alone: of many, the first, the last and some between)
+    rows = np.arange(nrow) if nrow < 500 else np.r_[0:40, nrow - 40:nrow, rng.integers(0, nrow, 200)]
+    got = out.cpu().numpy().reshape(nrow, -1)
+    assert np.array_equal(got[rows], oracle_lib.quantize(Q4_0, x[rows], im).reshape(len(rows), -1))
 
 
 @pytest.mark.parametrize("src", [F32, BF16], ids=["f32", "bf16"])
@@ -39,6 +42,10 @@ def test_rows(oracle_lib, src, nrow, ncol):
     run(oracle_lib, src, nrow, ncol)
 
 
-def test_many_rows(oracle_lib):
+@pytest.mark.parametrize("ncol", [384, 480, 512])
+@pytest.mark.parametrize("past", [0, 1])
+@pytest.mark.parametrize("a_cu", [32, 64])
+def test_many_rows(oracle_lib, a_cu, past, ncol):
+    """the row counts from which a lane takes a row: 32 a CU under 512 values, 64 from there (BF16)"""
     import torch
-    run(oracle_lib, BF16, 64 * torch.cuda.get_device_properties(0).multi_processor_count + 1, 384)
+    run(oracle_lib, BF16, a_cu * torch.cuda.get_device_properties(0).multi_processor_count + past, ncol)

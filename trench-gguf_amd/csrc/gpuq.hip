@@ -431,9 +431,12 @@ bool launch_rows(int type, int src, QParams p, int64_t rows, int64_t n_per_row, 
     if (rowsig_type(type) && p.qw) {
         // 16 rows a workgroup, or a lane a row where that fills the GPU or a row is shorter than one round. Microseconds
         // (lane, workgroup): 2048 rows of 7200 BF16 109, 32; 32768 of 1760 30, 39 (MXFP4 73, 47); 16384 of 3616 Q8_0
-        // 126, 37; 65536 of 384 BF16 10, 25; 4096 of 96 3.2, 3.5
-        const bool packed = src == T_Q8_0 || src == T_MXFP4;
-        const bool wg = n_per_row >= 32 * RSW_UNITS && rows <= (int64_t)g_ncu * (packed ? 128 : 64);
+        // 126, 37; 65536 of 384 BF16 10, 25; 4096 of 96 3.2, 3.5. Rows under 512 values of the two sources that a lane
+        // reads fastest gain from half as many at most (whole calls, lane and workgroup: 12000 of 416 BF16 48.2, 50.1 and
+        // 8192 34.4, 34.1; 32768 of 384 Q8_0 90.3, 93.2 and 16385 62.8, 61.7)
+        const bool packed = src == T_Q8_0 || src == T_MXFP4, quick = src == T_Q8_0 || src == T_BF16;
+        const int64_t most = (int64_t)g_ncu * (packed ? 128 : 64) / (quick && n_per_row < 512 ? 2 : 1);
+        const bool wg = n_per_row >= 32 * RSW_UNITS && rows <= most;
         const unsigned grid = (unsigned)(wg ? (rows + RSW_ROWS - 1) / RSW_ROWS : (rows + 255) / 256);
 #define KSIG(S)                                                                                             \
     if (wg)                                                                                                 \
