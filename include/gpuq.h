@@ -127,8 +127,9 @@ int gpuq_hessian_accumulate_dev(const float *d_X, int64_t nrows, int64_t ne0, do
  * normalized, block-permuted Hessian, with the reference's dead-column rule and its one retry with 10x more ridge),
  * perm [ne0] (host: the column permutation, whole 256-column blocks; order 0 'seq', 1 'act'), diag_n [ne0] (host,
  * diag(H)/n permuted; may be NULL) and dead [ne0] (host flags, original order; may be NULL).
- * Returns 0; 1 bad arguments (ne0 a multiple of 256, at most 65280), 3 not positive definite, 4 a HIP error.
- * Synchronizes `stream`. */
+ * Returns 0; 1 bad arguments (ne0 a multiple of 256, at most 65280), 3 not positive definite (of an ill-conditioned
+ * matrix also where its inverse is not, as the reference refuses it: such a call holds another ne0 x ne0 f64 matrix
+ * while it runs), 4 a HIP error. Synchronizes `stream`. */
 int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n, double damp, int order, double *d_U,
                              int64_t *perm, double *diag_n, unsigned char *dead, void *stream);
 

@@ -54,6 +54,39 @@ def test_factor(env, ne0):
     assert np.linalg.norm(U - want) <= tol * np.linalg.norm(want)
 
 
+def singular(n, seed):
+    """an exactly singular H: whole numbers, one column twice"""
+    rng = np.random.default_rng(seed)
+    X = rng.integers(-9, 10, (n + 64, n)).astype(np.float64)
+    j, k = rng.integers(0, n, 2)
+    X[:, j] = X[:, k]
+    return X.T @ X
+
+
+@pytest.mark.parametrize("ne0,seed", [(256, 6), (512, 0), (512, 5), (512, 8), (768, 8)])
+def test_factor_refuses_singular(env, ne0, seed):
+    """singular matrices that a factorization last column first lets pass (its last pivots are rounding errors above 0),
+    while one first column first, or that of the inverse, does not (the reference's, tools/ldlq.py:57-68): refused"""
+    print("case factor singular", ne0, seed, flush=True)
+    assert prepare(env, singular(ne0, seed), 1, damp=0.0)[0] == 3
+
+
+@pytest.mark.parametrize("ne0", [256, 768])
+@pytest.mark.parametrize("back", [False, True])
+def test_factor_of_a_graded_matrix(env, ne0, back):
+    """a condition of 1e24 that is scaling alone is no reason to refuse, and costs no accuracy: with A = D B D,
+    U D is B's factor's inverse"""
+    d = np.logspace(0, -12, ne0)[::-1 if back else 1]
+    i = np.arange(ne0)
+    B = np.eye(ne0) + 0.3 * np.exp(-abs(i[:, None] - i[None]) / 3.0)
+    print("case factor graded", ne0, back, flush=True)
+    rc, U = prepare(env, d[:, None] * B * d[None], 1, damp=0.0)
+    assert rc == 0
+    want, V = factor(B)
+    # (two factorizations as in test_factor, and the roundings of D B D)
+    assert np.linalg.norm(U * d - want) <= 3 * ne0 * 2.0 ** -53 * np.linalg.cond(V) * np.linalg.norm(want)
+
+
 def test_factor_retries_with_more_ridge_and_refuses(env):
     """Not positive definite with the ridge, but with ten times more: the retry's factor; with neither, or with a value
     that is not finite: 3"""

@@ -13,7 +13,7 @@
 //                    part of a step costs nothing while the rest of the matrix is large
 //   then U from the diagonal blocks' inverses by doubling: of neighbouring inverted runs of s blocks, U11 and U22, with
 //   V12 between them, U12 = -U11 (V12 U22) (k_tri_mul1, k_tri_mul2; the product in brackets goes, transposed, to the
-//   unused lower triangle), s = 1, 2, 4, ...; k_zero_lower clears the lower triangle at the end.
+//   unused lower triangle), s = 1, 2, 4, ...; k_upper_rows clears the lower triangle at the end.
 //
 // All products run on the f64 matrix cores. 7168 columns take 7.3 ms, where potrf, potri and potrf of rocSOLVER between
 // permutation and triangle kernels took 67.6 ms (26 ms of it in their serial 128-column kernels): 56 steps of 48 to 164 us
@@ -545,8 +545,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     G::each(acc, [&](int r, int c, double v) { o[(int64_t)r * n + c] = v; });
 }
 
-// zero the strict lower triangle; grid (ceil(n / 256), n)
-__global__ __launch_bounds__(256) void k_zero_lower(double *__restrict__ A, int64_t n) {
-    const int64_t i = blockIdx.y, j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (j < i) A[i * n + j] = 0.0;
+// zero the strict lower triangle and sum the squares of each row's rest (a row a workgroup): the trace of U^T U, by which
+// the caller sees whether A was so ill-conditioned that the reference's route has to be asked (gpuq_prepare_hessian_dev)
+__global__ __launch_bounds__(256) void k_upper_rows(double *__restrict__ A, int64_t n, double *__restrict__ sq) {
+    __shared__ double part[4];
+    const int64_t i = blockIdx.x;
+    double *row = A + i * n, s = 0.0;
+    for (int64_t j = threadIdx.x; j < i; j += 256) row[j] = 0.0;
+#pragma unroll 4
+    for (int64_t j = (i & ~255ll) + threadIdx.x; j < n; j += 256) {
+        const double v = row[j];
+        s = fma(v, j < i ? 0.0 : v, s);
+    }
+    for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
+    if (lane_id() == 0) part[wave_id()] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) sq[i] = part[0] + part[1] + part[2] + part[3];
+}
+
+// X = U^T U read backwards (row i of R is row n-1-i of X), the 128-blocks of its upper triangle; grid nb(nb+1)/2
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_utu_reversed(const double *__restrict__ U,
+                                                                                             int64_t n,
+                                                                                             double *__restrict__ R) {
+    using G = ChTile<CH_NB, CH_NB, 2, true, true>;
+    __shared__ __align__(16) double lds[G::LDS];
+    const int64_t t = blockIdx.x;
+    int64_t p = (int64_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+    while (p * (p + 1) / 2 > t) --p;
+    while ((p + 1) * (p + 2) / 2 <= t) ++p;
+    const int64_t q = t - p * (p + 1) / 2;               // blocks q <= p of X: its lower triangle, R's upper one
+    ldlq_d4 acc[G::MI][G::NJ];
+    G::zero(acc);
+    G::template product<false>(U + p * CH_NB, n, U + q * CH_NB, n, (int)(q + 1) * CH_NB, lds, acc);
+    double *o = R + (n - 1 - p * CH_NB) * n + n - 1 - q * CH_NB;
+    G::each(acc, [&](int r, int c, double v) { o[-(int64_t)r * n - c] = v; });
 }

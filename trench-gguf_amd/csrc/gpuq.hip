@@ -1084,33 +1084,48 @@ extern "C" size_t gpuq_ldlq_dev_noalloc(int type, float *d_wp, const double *d_u
 namespace {
 
 std::mutex g_mu_h;   // the Hessian preparation's buffer
-Buf g_hd;            // device: diag (f64) | perm (i64) | dead (u8) | factorization info
+Buf g_hd;            // device: diag, then the rows' squares (f64) | factorization info (8 bytes) | perm (i64) | dead (u8)
+struct Scratch {     // device memory of one call
+    void *p = nullptr;
+    ~Scratch() {
+        if (p) (void)hipFree(p);
+    }
+};
 
-// U (chol.cuh) in place of the permuted Hessian A (its upper triangle), launches only; *d_info (zeroed by the caller)
-// becomes 1 when A is not positive definite
-void launch_factor(double *A, int64_t n, int *d_info, hipStream_t st) {
-    const int64_t nb = n / CH_NB;
+// A = V V^T (chol.cuh) in place on A's upper triangle, the diagonal blocks inverted, launches only; *d_info becomes 1 when
+// A is not positive definite
+void launch_chol(double *A, int64_t n, int *d_info, hipStream_t st) {
+    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, d_info);
     hipLaunchKernelGGL(k_chol_last, dim3(1), dim3(256), 0, st, A, n, d_info);
-    for (int64_t k = nb - 1; k > 0; --k) {
+    for (int64_t k = n / CH_NB - 1; k > 0; --k) {
         hipLaunchKernelGGL(k_chol_panel, dim3((unsigned)(k * CH_NB / 32)), dim3(256), 0, st, A, n, k);
         const int64_t nt = k * (k + 1) / 2 - 1;          // the tiles beside (k-1, k-1), in whole rounds of the 8 XCDs
         hipLaunchKernelGGL(k_chol_update, dim3((unsigned)(1 + (nt + 7) / 8 * 8)), dim3(256), 0, st, A, n, k, d_info);
     }
+}
+
+// U = V^-1 from there, and the sums of its rows' squares
+void launch_inverse(double *A, int64_t n, double *d_sq, hipStream_t st) {
+    const int64_t nb = n / CH_NB;
     for (int64_t s = 1; s < nb; s *= 2) {
         const int64_t pairs = (nb - s + 2 * s - 1) / (2 * s), t = s * (CH_NB / CHT);
         const dim3 grid((unsigned)(t * t), (unsigned)pairs);
         hipLaunchKernelGGL(k_tri_mul1, grid, dim3(256), 0, st, A, n, s);
         hipLaunchKernelGGL(k_tri_mul2, grid, dim3(256), 0, st, A, n, s);
     }
-    hipLaunchKernelGGL(k_zero_lower, dim3((unsigned)((n + 255) / 256), (unsigned)n), dim3(256), 0, st, A, n);
+    hipLaunchKernelGGL(k_upper_rows, dim3((unsigned)n), dim3(256), 0, st, A, n, d_sq);
 }
 
-// a factorization's info (0: done; > 0: not positive definite), -1 when it cannot be read
-int read_info(const int *d_info, hipStream_t st) {
-    int v = -1;
-    if (hipMemcpyAsync(&v, d_info, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
+// a factorization's rows' squares and info (0: done; > 0: not positive definite), one after the other on the device;
+// -1 when they cannot be read
+int read_factor(const double *d_sq, int64_t n, std::vector<double> &sq, hipStream_t st) {
+    sq.resize((size_t)n + 1);
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(sq.data(), d_sq, (size_t)(n + 1) * 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return -1;
+    int v;
+    memcpy(&v, &sq[(size_t)n], sizeof(int));
     return v;
 }
 
@@ -1139,15 +1154,15 @@ extern "C" int gpuq_hessian_accumulate_dev(const float *d_X, int64_t nrows, int6
 // rows; one retry with 10x more ridge when Hp does not factor), and on the host perm (ne0 column indices, whole
 // 256-blocks: order 0 'seq' keeps them in order, 1 'act' sorts them by descending energy, ties in order), diag_n
 // (diag(Hn)[perm]) and dead (ne0 flags, original order); either of the last two may be NULL. Returns 0, or 1 for bad
-// arguments, 3 when the matrix does not factor, 4 on a HIP error.
+// arguments, 3 when the matrix (or, where it is ill-conditioned, its inverse) does not factor, 4 on a HIP error.
 extern "C" int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n, double damp, int order, double *d_U,
                                         int64_t *perm, double *diag_n, uint8_t *dead, void *stream) {
     if (g_device < 0 || !d_H || !d_U || !perm || ne0 <= 0 || ne0 % QK || ne0 > 65535) return 1;   // (grid rows)
     if ((order != 0 && order != 1) || !(damp >= 0) || ((uintptr_t)d_H & 7) || ((uintptr_t)d_U & 7)) return 1;
     std::lock_guard<std::mutex> lock(g_mu_h);
     const hipStream_t st = (hipStream_t)stream;
-    const size_t o_perm = (size_t)ne0 * 8, o_dead = o_perm + (size_t)ne0 * 8, o_info = (o_dead + ne0 + 15) & ~15ull;
-    if (!g_hd.grow(o_info + 16)) return 4;
+    const size_t o_info = (size_t)ne0 * 8, o_perm = o_info + 8, o_dead = o_perm + (size_t)ne0 * 8;
+    if (!g_hd.grow(o_dead + (size_t)ne0)) return 4;
     double *dd = (double *)g_hd.p;
     int64_t *dp = (int64_t *)((uint8_t *)g_hd.p + o_perm);
     uint8_t *dz = (uint8_t *)g_hd.p + o_dead;
@@ -1187,19 +1202,44 @@ extern "C" int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n
     if (hipMemcpyAsync(dp, pm.data(), (size_t)ne0 * 8, hipMemcpyHostToDevice, st) != hipSuccess ||
         hipMemcpyAsync(dz, zd.data(), (size_t)ne0, hipMemcpyHostToDevice, st) != hipSuccess)
         return 4;
-    const double r1 = damp * mean;
-    int info = 0;
-    for (int tries = 0; tries < 2; ++tries) {             // (the second: more ridge until it factors)
+    const double r1 = damp * mean, r2 = 10 * damp * mean;
+    // the permuted matrix, with the second try's ridge (more until it factors); with rev read backwards
+    auto build = [&](int tries, bool rev, double *A) {
         hipLaunchKernelGGL(k_hess_perm, g2, dim3(256), 0, st, d_H, ne0, nd, (const int64_t *)dp, (const uint8_t *)dz, r1,
-                           d_U);
-        if (tries) hipLaunchKernelGGL(k_diag_add, dim3(g1), dim3(256), 0, st, d_U, ne0, 10 * damp * mean);
-        hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, dinfo);
-        launch_factor(d_U, ne0, dinfo, st);
-        if (hipGetLastError() != hipSuccess) return 4;
-        info = read_info(dinfo, st);
-        if (info <= 0) break;
+                           rev, A);
+        if (tries) hipLaunchKernelGGL(k_diag_add, dim3(g1), dim3(256), 0, st, A, ne0, r2);
+    };
+    std::vector<double> sq;
+    Scratch x;                                            // (the ill-conditioned matrices' second matrix)
+    int info = 0;
+    for (int tries = 0; tries < 2; ++tries) {
+        build(tries, false, d_U);
+        launch_chol(d_U, ne0, dinfo, st);
+        launch_inverse(d_U, ne0, dd, st);
+        if ((info = read_factor(dd, ne0, sq, st)) < 0) return 4;
+        if (info > 0) continue;
+        // The reference factors the matrix first column first and then its inverse, and refuses a matrix whose inverse does
+        // not factor. The inverse, formed in f64 and factored, is off by less than (2n + 2) u trace(A^-1) (N. Higham,
+        // Accuracy and Stability of Numerical Algorithms, theorem 10.3), so it factors where that is below its least
+        // eigenvalue, 1 / trace(A) at least; the matrix likewise. Other matrices are put to both factorizations.
+        double ta = (double)ne0 * (r1 + (tries ? r2 : 0)), tx = 0;
+        for (int64_t i = 0; i < ne0; ++i) {
+            ta += d[i];
+            tx += sq[i];
+        }
+        if (ta * tx * 4.0 * (double)ne0 * 0x1p-53 < 1.0) break;
+        if (!x.p && hipMalloc(&x.p, (size_t)ne0 * ne0 * 8) != hipSuccess) return 4;
+        build(tries, true, (double *)x.p);
+        launch_chol((double *)x.p, ne0, dinfo, st);
+        if ((info = read_factor(dd, ne0, sq, st)) < 0) return 4;
+        if (info > 0) continue;
+        const int64_t nb = ne0 / CH_NB;
+        hipLaunchKernelGGL(k_utu_reversed, dim3((unsigned)(nb * (nb + 1) / 2)), dim3(256), 0, st, d_U, ne0, (double *)x.p);
+        launch_chol((double *)x.p, ne0, dinfo, st);
+        if ((info = read_factor(dd, ne0, sq, st)) < 0) return 4;
+        break;
     }
-    if (info != 0) return info > 0 ? 3 : 4;
+    if (info) return 3;
     for (int64_t i = 0; i < ne0; ++i) {
         perm[i] = pm[i];
         if (diag_n) diag_n[i] = d[pm[i]];
