@@ -7,6 +7,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 Q4_K = 12
+LDLQ_TYPES = {16: "iq2_xxs", 17: "iq2_xs", 22: "iq2_s", 18: "iq3_xxs", 21: "iq3_s", 19: "iq1_s", 29: "iq1_m", 23: "iq4_xs",
+              10: "q2_k", 11: "q3_k", 12: "q4_k", 13: "q5_k", 14: "q6_k"}
 
 
 @pytest.fixture(scope="module")
@@ -50,20 +52,31 @@ def test_rows(env, oracle_lib, nmat, ne1, own):
     check(env, oracle_lib, Q4_K, W, U, own)
 
 
-def test_rows_either_side(env):
-    """a matrix alone (16 rows a workgroup) and the same among many (64 rows a wave) give the same bytes"""
+@pytest.mark.parametrize("typ", list(LDLQ_TYPES), ids=list(LDLQ_TYPES.values()))
+def test_rows_either_side(env, oracle_lib, typ):
+    """a stack of ragged matrices with more than five groups of 16 rows a CU (64 rows a wave, 128 x 128 update tiles), one
+    matrix fewer (16 rows a workgroup) and few enough for 64 x 64 tiles: the same bytes, and the oracle's in sampled rows"""
     torch, gq = env
     from gpuq import ldlq
     rng = np.random.default_rng(5)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    nmat, ne1, ne0 = 5 * cus // 6 + 1, 90, 512                # 6 groups of 16 rows a matrix: just over 5 a CU
-    U = torch.from_numpy(factor(rng, ne0)).cuda()
+    nmat, ne1, ne0 = 5 * cus // 6 + 1, 90, 768                # 6 groups of 16 rows a matrix: just over 5 a CU
+    few = cus // 4                                            # 4 tiles of 128 x 128 in two blocks, 2 in one
+    U = factor(rng, ne0)
+    dU = torch.from_numpy(U).cuda()
     W = torch.randn(nmat, ne1, ne0, device="cuda", generator=torch.Generator("cuda").manual_seed(1)) * 0.05
-    qw = torch.ones(nmat, ne0, device="cuda")
+    qw = rng.lognormal(0, 1, (nmat, ne0)).astype(np.float32)
+    dqw = torch.from_numpy(qw).cuda()
     perm = np.arange(ne0)
-    many = ldlq.quantize_matrix_dev(gq, Q4_K, W, U, perm, qw).clone()
-    fewer = ldlq.quantize_matrix_dev(gq, Q4_K, W[:-1].contiguous(), U, perm, qw[:-1].contiguous()).clone()
-    assert torch.equal(many[:-1], fewer)
+    print("case ldlq either side %s" % LDLQ_TYPES[typ], flush=True)
+    many = ldlq.quantize_matrix_dev(gq, typ, W, dU, perm, dqw).clone()
+    for n in (nmat - 1, few - 1):
+        fewer = ldlq.quantize_matrix_dev(gq, typ, W[:n].contiguous(), dU, perm, dqw[:n].contiguous())
+        assert torch.equal(many[:n], fewer), n
+    rows = [0, 15, 63, 64, 80, 89]
+    for m in (0, nmat // 2, nmat - 1):
+        want = oracle_lib.ldlq(typ, W[m:m + 1, rows].cpu().numpy(), U, qw[m:m + 1], ldlq.slot_order(perm))[0]
+        assert np.array_equal(many[m, rows].cpu().numpy().reshape(-1), want.reshape(-1)), m
 
 
 @pytest.mark.parametrize("what", ["zero rows", "large factor", "small factor", "zero diagonal", "infinite weight"])
