@@ -50,8 +50,10 @@ def test_factor(env, ne0):
     assert rc == 0
     assert np.array_equal(np.tril(U, -1), np.zeros_like(U))
     # first-order bound of both factorizations: each off by at most n u cond(V) relative
-    tol = 2 * ne0 * 2.0 ** -53 * np.linalg.cond(V)
-    assert np.linalg.norm(U - want) <= tol * np.linalg.norm(want)
+    rel = np.linalg.norm(U - want) / np.linalg.norm(want)
+    assert rel <= 2 * ne0 * 2.0 ** -53 * np.linalg.cond(V)
+    # and four times what these well-conditioned inputs (cond(V) 7 to 20) measure, n u / 90: 3.2e-16 to 2.4e-15
+    assert rel <= ne0 * 2.0 ** -53 / 22
 
 
 def singular(n, seed):
