@@ -545,9 +545,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     G::each(acc, [&](int r, int c, double v) { o[(int64_t)r * n + c] = v; });
 }
 
-// zero the strict lower triangle and sum the squares of each row's rest (a row a workgroup): the trace of U^T U, by which
-// the caller sees whether A was so ill-conditioned that the reference's route has to be asked (gpuq_prepare_hessian_dev)
-__global__ __launch_bounds__(256) void k_upper_rows(double *__restrict__ A, int64_t n, double *__restrict__ sq) {
+// Zero the strict lower triangle and add up the squares of the rest, a row a workgroup: the trace of U^T U, by which the
+// caller sees whether A was so ill-conditioned that the reference's route has to be asked (gpuq_prepare_hessian_dev). The
+// rows' sums go to CH_SUMS sums, in any order: the rule that reads them leaves more room than that makes. 56 us at 7168
+// columns, and 48 without the squares.
+#define CH_SUMS 64
+__global__ __launch_bounds__(256) void k_upper_rows(double *__restrict__ A, int64_t n, double *__restrict__ sums) {
     __shared__ double part[4];
     const int64_t i = blockIdx.x;
     double *row = A + i * n, s = 0.0;
@@ -560,16 +563,19 @@ __global__ __launch_bounds__(256) void k_upper_rows(double *__restrict__ A, int6
     for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
     if (lane_id() == 0) part[wave_id()] = s;
     __syncthreads();
-    if (threadIdx.x == 0) sq[i] = part[0] + part[1] + part[2] + part[3];
+    if (threadIdx.x == 0) atomicAdd(sums + i % CH_SUMS, part[0] + part[1] + part[2] + part[3]);
 }
 
-// X = U^T U read backwards (row i of R is row n-1-i of X), the 128-blocks of its upper triangle; grid nb(nb+1)/2
+// X = U^T U read backwards (row i of R is row n-1-i of X), the 128-blocks of its upper triangle; grid nb(nb+1)/2. The first
+// workgroup clears what the factorization adds to (nz <= 256 doubles)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_utu_reversed(const double *__restrict__ U,
                                                                                              int64_t n,
-                                                                                             double *__restrict__ R) {
+                                                                                             double *__restrict__ R,
+                                                                                             double *__restrict__ z, int nz) {
     using G = ChTile<CH_NB, CH_NB, 2, true, true>;
     __shared__ __align__(16) double lds[G::LDS];
     const int64_t t = blockIdx.x;
+    if (t == 0 && (int)threadIdx.x < nz) z[threadIdx.x] = 0.0;
     int64_t p = (int64_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
     while (p * (p + 1) / 2 > t) --p;
     while ((p + 1) * (p + 2) / 2 <= t) ++p;

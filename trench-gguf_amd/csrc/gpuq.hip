@@ -1084,7 +1084,7 @@ extern "C" size_t gpuq_ldlq_dev_noalloc(int type, float *d_wp, const double *d_u
 namespace {
 
 std::mutex g_mu_h;   // the Hessian preparation's buffer
-Buf g_hd;            // device: diag, then the rows' squares (f64) | factorization info (8 bytes) | perm (i64) | dead (u8)
+Buf g_hd;            // device: diag (f64) | a factorization's result (FACTOR_RESULT f64) | perm (i64) | dead (u8)
 struct Scratch {     // device memory of one call
     void *p = nullptr;
     ~Scratch() {
@@ -1092,10 +1092,14 @@ struct Scratch {     // device memory of one call
     }
 };
 
-// A = V V^T (chol.cuh) in place on A's upper triangle, the diagonal blocks inverted, launches only; *d_info becomes 1 when
-// A is not positive definite
-void launch_chol(double *A, int64_t n, int *d_info, hipStream_t st) {
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, d_info);
+// what a factorization leaves on the device: U's squares (CH_SUMS sums) and its info (8 bytes, an int)
+constexpr int FACTOR_RESULT = CH_SUMS + 1;
+int *factor_info(double *d_res) { return (int *)(d_res + CH_SUMS); }
+
+// A = V V^T (chol.cuh) in place on A's upper triangle, the diagonal blocks inverted, launches only; the result, cleared
+// by the kernel that built A, gets info 1 when A is not positive definite
+void launch_chol(double *A, int64_t n, double *d_res, hipStream_t st) {
+    int *d_info = factor_info(d_res);
     hipLaunchKernelGGL(k_chol_last, dim3(1), dim3(256), 0, st, A, n, d_info);
     for (int64_t k = n / CH_NB - 1; k > 0; --k) {
         hipLaunchKernelGGL(k_chol_panel, dim3((unsigned)(k * CH_NB / 32)), dim3(256), 0, st, A, n, k);
@@ -1104,8 +1108,8 @@ void launch_chol(double *A, int64_t n, int *d_info, hipStream_t st) {
     }
 }
 
-// U = V^-1 from there, and the sums of its rows' squares
-void launch_inverse(double *A, int64_t n, double *d_sq, hipStream_t st) {
+// U = V^-1 from there, and the sums of its squares
+void launch_inverse(double *A, int64_t n, double *d_res, hipStream_t st) {
     const int64_t nb = n / CH_NB;
     for (int64_t s = 1; s < nb; s *= 2) {
         const int64_t pairs = (nb - s + 2 * s - 1) / (2 * s), t = s * (CH_NB / CHT);
@@ -1113,19 +1117,20 @@ void launch_inverse(double *A, int64_t n, double *d_sq, hipStream_t st) {
         hipLaunchKernelGGL(k_tri_mul1, grid, dim3(256), 0, st, A, n, s);
         hipLaunchKernelGGL(k_tri_mul2, grid, dim3(256), 0, st, A, n, s);
     }
-    hipLaunchKernelGGL(k_upper_rows, dim3((unsigned)n), dim3(256), 0, st, A, n, d_sq);
+    hipLaunchKernelGGL(k_upper_rows, dim3((unsigned)n), dim3(256), 0, st, A, n, d_res);
 }
 
-// a factorization's rows' squares and info (0: done; > 0: not positive definite), one after the other on the device;
-// -1 when they cannot be read
-int read_factor(const double *d_sq, int64_t n, std::vector<double> &sq, hipStream_t st) {
-    sq.resize((size_t)n + 1);
+// a factorization's info (0: done; > 0: not positive definite) and the sum of U's squares; -1 when they cannot be read
+int read_factor(const double *d_res, double &squares, hipStream_t st) {
+    double res[FACTOR_RESULT];
     if (hipGetLastError() != hipSuccess ||
-        hipMemcpyAsync(sq.data(), d_sq, (size_t)(n + 1) * 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipMemcpyAsync(res, d_res, sizeof res, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return -1;
+    squares = 0;
+    for (int i = 0; i < CH_SUMS; ++i) squares += res[i];
     int v;
-    memcpy(&v, &sq[(size_t)n], sizeof(int));
+    memcpy(&v, res + CH_SUMS, sizeof v);
     return v;
 }
 
@@ -1161,12 +1166,12 @@ extern "C" int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n
     if ((order != 0 && order != 1) || !(damp >= 0) || ((uintptr_t)d_H & 7) || ((uintptr_t)d_U & 7)) return 1;
     std::lock_guard<std::mutex> lock(g_mu_h);
     const hipStream_t st = (hipStream_t)stream;
-    const size_t o_info = (size_t)ne0 * 8, o_perm = o_info + 8, o_dead = o_perm + (size_t)ne0 * 8;
+    const size_t o_perm = (size_t)(ne0 + FACTOR_RESULT) * 8, o_dead = o_perm + (size_t)ne0 * 8;
     if (!g_hd.grow(o_dead + (size_t)ne0)) return 4;
     double *dd = (double *)g_hd.p;
     int64_t *dp = (int64_t *)((uint8_t *)g_hd.p + o_perm);
     uint8_t *dz = (uint8_t *)g_hd.p + o_dead;
-    int *dinfo = (int *)((uint8_t *)g_hd.p + o_info);
+    double *dres = dd + ne0;
     const double nd = 1.0 > n ? 1.0 : n;                       // max(n, 1)
     const unsigned g1 = (unsigned)((ne0 + 255) / 256);
     const dim3 g2(g1, (unsigned)ne0);
@@ -1203,40 +1208,38 @@ extern "C" int gpuq_prepare_hessian_dev(const double *d_H, int64_t ne0, double n
         hipMemcpyAsync(dz, zd.data(), (size_t)ne0, hipMemcpyHostToDevice, st) != hipSuccess)
         return 4;
     const double r1 = damp * mean, r2 = 10 * damp * mean;
-    // the permuted matrix, with the second try's ridge (more until it factors); with rev read backwards
-    auto build = [&](int tries, bool rev, double *A) {
-        hipLaunchKernelGGL(k_hess_perm, g2, dim3(256), 0, st, d_H, ne0, nd, (const int64_t *)dp, (const uint8_t *)dz, r1,
-                           rev, A);
+    // the permuted matrix, with the second try's ridge (more until it factors)
+    auto build = [&](decltype(&k_hess_perm<false>) perm_kernel, int tries, double *A) {
+        hipLaunchKernelGGL(perm_kernel, g2, dim3(256), 0, st, d_H, ne0, nd, (const int64_t *)dp, (const uint8_t *)dz, r1, A,
+                           dres, FACTOR_RESULT);
         if (tries) hipLaunchKernelGGL(k_diag_add, dim3(g1), dim3(256), 0, st, A, ne0, r2);
     };
-    std::vector<double> sq;
+    double tx = 0;                                        // trace(A^-1): the sum of U's squares
     Scratch x;                                            // (the ill-conditioned matrices' second matrix)
     int info = 0;
     for (int tries = 0; tries < 2; ++tries) {
-        build(tries, false, d_U);
-        launch_chol(d_U, ne0, dinfo, st);
-        launch_inverse(d_U, ne0, dd, st);
-        if ((info = read_factor(dd, ne0, sq, st)) < 0) return 4;
+        build(k_hess_perm<false>, tries, d_U);
+        launch_chol(d_U, ne0, dres, st);
+        launch_inverse(d_U, ne0, dres, st);
+        if ((info = read_factor(dres, tx, st)) < 0) return 4;
         if (info > 0) continue;
         // The reference factors the matrix first column first and then its inverse, and refuses a matrix whose inverse does
         // not factor. The inverse, formed in f64 and factored, is off by less than (2n + 2) u trace(A^-1) (N. Higham,
         // Accuracy and Stability of Numerical Algorithms, theorem 10.3), so it factors where that is below its least
         // eigenvalue, 1 / trace(A) at least; the matrix likewise. Other matrices are put to both factorizations.
-        double ta = (double)ne0 * (r1 + (tries ? r2 : 0)), tx = 0;
-        for (int64_t i = 0; i < ne0; ++i) {
-            ta += d[i];
-            tx += sq[i];
-        }
+        double ta = (double)ne0 * (r1 + (tries ? r2 : 0));
+        for (int64_t i = 0; i < ne0; ++i) ta += d[i];
         if (ta * tx * 4.0 * (double)ne0 * 0x1p-53 < 1.0) break;
         if (!x.p && hipMalloc(&x.p, (size_t)ne0 * ne0 * 8) != hipSuccess) return 4;
-        build(tries, true, (double *)x.p);
-        launch_chol((double *)x.p, ne0, dinfo, st);
-        if ((info = read_factor(dd, ne0, sq, st)) < 0) return 4;
+        build(k_hess_perm<true>, tries, (double *)x.p);     // (read backwards: first column first)
+        launch_chol((double *)x.p, ne0, dres, st);
+        if ((info = read_factor(dres, tx, st)) < 0) return 4;
         if (info > 0) continue;
         const int64_t nb = ne0 / CH_NB;
-        hipLaunchKernelGGL(k_utu_reversed, dim3((unsigned)(nb * (nb + 1) / 2)), dim3(256), 0, st, d_U, ne0, (double *)x.p);
-        launch_chol((double *)x.p, ne0, dinfo, st);
-        if ((info = read_factor(dd, ne0, sq, st)) < 0) return 4;
+        hipLaunchKernelGGL(k_utu_reversed, dim3((unsigned)(nb * (nb + 1) / 2)), dim3(256), 0, st, d_U, ne0, (double *)x.p,
+                           dres, FACTOR_RESULT);
+        launch_chol((double *)x.p, ne0, dres, st);
+        if ((info = read_factor(dres, tx, st)) < 0) return 4;
         break;
     }
     if (info) return 3;

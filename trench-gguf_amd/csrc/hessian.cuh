@@ -12,21 +12,19 @@ __global__ __launch_bounds__(256) void k_hess_diag(const double *__restrict__ H,
 }
 
 // Hp[i][j] = Hn[perm[i]][perm[j]] (a dead column's row and column zero, its diagonal 1), plus ridge on the diagonal, for
-// the 128-blocks of the upper triangle (all that the factorization reads); with rev Hp read backwards, from the same
-// entries of H; grid (ceil(ne0 / 256), ne0)
+// the 128-blocks of the upper triangle (all that the factorization reads); with REV Hp read backwards, from the same
+// entries of H; grid (ceil(ne0 / 256), ne0). The first workgroup clears what the factorization adds to (nz <= 256 doubles)
+template <bool REV>
 __global__ __launch_bounds__(256) void k_hess_perm(const double *__restrict__ H, int64_t ne0, double nd,
                                                    const int64_t *__restrict__ perm, const uint8_t *__restrict__ dead,
-                                                   double ridge, bool rev, double *__restrict__ Hp) {
+                                                   double ridge, double *__restrict__ Hp, double *__restrict__ z, int nz) {
     const int64_t i = blockIdx.y, j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i == 0 && blockIdx.x == 0 && (int)threadIdx.x < nz) z[threadIdx.x] = 0.0;
     if (j >= ne0 || j / 128 < i / 128) return;
-    const int64_t pi = perm[rev ? ne0 - 1 - j : i], pj = perm[rev ? ne0 - 1 - i : j];
+    const int64_t pi = perm[REV ? ne0 - 1 - j : i], pj = perm[REV ? ne0 - 1 - i : j];
     double v = dead[pi] || dead[pj] ? (pi == pj ? 1.0 : 0.0) : H[pi * ne0 + pj] / nd;
     if (i == j) v += ridge;
     Hp[i * ne0 + j] = v;
-}
-
-__global__ void k_zero_int(int *v) {
-    if (threadIdx.x == 0) *v = 0;
 }
 
 // A[i][i] += r
