@@ -100,7 +100,7 @@ def prepare_dev(torch, gq, H, n, order, damp=0.01):
 
 @pytest.mark.parametrize("order", ["seq", "act"])
 def test_prepare_hessian_dev_matches_host(env, order):
-    """the device factor (rocSOLVER potrf / potri) against the host restatement of tools/ldlq.py:34-68: the same
+    """the device factor (csrc/chol.cuh) against the host restatement of tools/ldlq.py:34-68: the same
     permutation, diag and dead columns exactly, the same U to rounding, and U^T U = (Hp + ridge)^-1"""
     torch, gpuq, gq = env
     from gpuq import ldlq

@@ -387,8 +387,9 @@ __global__ __launch_bounds__(256) void k_chol_panel(double *__restrict__ A, int6
     G::each(acc, [&](int r, int c, double v) { P[(int64_t)r * n + c] = v; });
 }
 
-// A[i][j] -= V[i][k] V[j][k]^T for the blocks i <= j < k; grid k(k+1)/2, workgroup 0 the block (k-1, k-1), which it also
-// factors. The other tiles are numbered column by column and dealt to the 8 XCDs in contiguous runs.
+// A[i][j] -= V[i][k] V[j][k]^T for the blocks i <= j < k; workgroup 0 takes the block (k-1, k-1), which it also factors, and
+// the rest of the grid (k(k+1)/2 - 1 rounded up to a multiple of 8) the other tiles, numbered column by column and dealt to
+// the 8 XCDs in contiguous runs.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_chol_update(double *__restrict__ A,
                                                                                             int64_t n, int64_t k,
                                                                                             int *__restrict__ info) {

@@ -7,10 +7,12 @@
 // order-free reductions (max). A wave therefore quantizes 64/G super-blocks at once, with 100% lane occupancy in the
 // fixed-trip-count search loops. Each wave assembles its super-blocks' output bytes in an LDS image and writes them
 // to HBM as one contiguous, dword-coalesced range. For the types with neighbour searches (tiles of varying cost) the
-// launch holds as many workgroups as the CUs keep resident, and each wave takes its tiles (64/G super-blocks, fewer in
-// calls that would leave waves without one) one at a time from a counter, unless each has its only one from the start: the waves sweep the tensor once, in order (an expert's importance row is read while the
-// whole chip works on that expert), every wave busy until the counter runs past the end. The other types loop over
-// the tiles grid-stride. The per-workgroup LDS table staging of the i-quants is paid once per workgroup.
+// launch holds as many workgroups as the CUs keep resident, and where the tiles (64/G super-blocks) outnumber their waves,
+// each wave takes its next chunk of tiles from a counter: the waves sweep the tensor once, in order (an expert's importance
+// row is read while the whole chip works on that expert), every wave busy until the counter runs past the end. A chunk is one
+// tile, or for the packed sources the tiles of a whole run of lines (KT), which one wave takes in turn, also where other
+// waves have none. Calls of few super-blocks have thinner tiles, one a wave (TH). The other types loop over the tiles
+// grid-stride. The per-workgroup LDS table staging of the i-quants is paid once per workgroup.
 #pragma once
 #include "common.cuh"
 
@@ -35,7 +37,8 @@ struct QParams {
     int *err;               // set when a search finds no candidate (the reference traps there)
     // the launch's tile counter (zeroed on the stream before the launch): after its first chunk of tiles (its wave
     // number) each wave takes the next from it (grid waves + the counter's old value), so the resident waves sweep
-    // the tensor once, in order, and finish together; nullptr: a fixed grid-stride order
+    // the tensor once, in order, and finish together; nullptr: a fixed grid-stride order (no wave has a second chunk,
+    // or gpuq_init has not run)
     unsigned long long *tiles;
     // strided views (the LDLQ loop quantizes one block column of every row): unit b reads its weights at element
     // b*sb_stride + sb_off, its importance at row*qw_stride + qw_off, and writes its block at byte
